@@ -809,7 +809,7 @@ __global__ __launch_bounds__(kBlock) void k_volt4(const GridDesc g, const QBoxes
     const unsigned long long pz = z0 ? p - g.plane : p;
     float4 Ix_zm = *reinterpret_cast<const float4*>(Ix + pz), Iy_zm = *reinterpret_cast<const float4*>(Iy + pz);
     // voltage sources added here (per-quad lists ordered by plane) where no
-    // hook sits between the update and the excitation; else by k_excite
+    // hook sits between the update and the excitation; else by the Excite hook
     SrcCursor cv{0u, 0u, ~0u};
     int ts = 0;
     if (ex.beg) {
@@ -1506,7 +1506,7 @@ __global__ __launch_bounds__(kBlock) void k_step2(const Step2Args a, const float
 struct MurFold {
     const float* cP;               // coefficients of the y and z components
     const float* cPP;
-    float* mP;                     // the hooks' values, read by k_mur_apply
+    float* mP;                     // the hooks' values, read by the MurApply hook
     float* mPP;
     unsigned start_ts;
     unsigned on;
@@ -1775,7 +1775,7 @@ __global__ __launch_bounds__(kBlock) void k_step4(const Step4Args ag, const floa
 constexpr unsigned kQTileRows = kBlock / 64;
 
 // Mur pre and post hooks of point k (coefficients cp, cpp) for face element
-// F and neighbour element S of a quad (k_mur_pre / k_mur_post arithmetic):
+// F and neighbour element S of a quad (the MurPre / MurPost hooks' arithmetic):
 // y and z from V^n (v0) and V^{n+1} (v); stored when `keep`
 template <int F, int S>
 __device__ __forceinline__ void mur_fold_quad(const MurFold& M, unsigned k, float cp, float cpp, const float4 v0[3],
@@ -1845,7 +1845,7 @@ __global__ __launch_bounds__(kBlock, 3) void k_step4t(const Step4Args ag, const 
     // the apply hook will set for the face's y and z components in its own
     // current update; it stores that value too, except on the face's rim,
     // where the other faces' hooks still read or write, and which
-    // k_mur_apply_rim sets afterwards
+    // the MurApply hook sets afterwards
     const bool flo = a.mf[0].on && x0 == 0 && (unsigned)ts >= a.mf[0].start_ts;
     const bool fhi = a.mf[1].on && x0 + 4 == Nx && (unsigned)ts >= a.mf[1].start_ts;
     SrcCursor cv = src_cursor(a.eV, evb, eve, z0), ci = src_cursor(a.eI, eib, eie, z0);
@@ -1919,7 +1919,7 @@ __global__ __launch_bounds__(kBlock, 3) void k_step4t(const Step4Args ag, const 
             quad_coef_n<CC>(a.kV, cs, p, u, 2, c, w);
             v[2] = quad_math(v0[2], c, w, quad_curl(iy, iy_xm, ix, ix_ym));
             quad_sources_at(a.eV, cv, x0, z, 7u, ts, v);
-            // the hook values are kept for k_mur_apply_rim on the face's rim
+            // the hook values are kept for the MurApply hook on the face's rim
             const bool keep = active && z < z1 && (y < 2 || y + 2 >= a.ny || z < 2 || z + 2 >= a.zb);
             if (flo) mur_fold_quad<0, 1>(a.mf[0], z * a.ny + y, mcp, mcpp, v0, v, keep, fy, fz);
             else if (fhi) mur_fold_quad<3, 2>(a.mf[1], z * a.ny + y, mcp, mcpp, v0, v, keep, fy, fz);
@@ -1935,7 +1935,7 @@ __global__ __launch_bounds__(kBlock, 3) void k_step4t(const Step4Args ag, const 
         }
         if (active && z < z1) {
             // face points off the face's rim (no other face's hook reads or
-            // writes them) are stored with the apply's value; k_mur_apply_rim
+            // writes them) are stored with the apply's value; the MurApply hook
             // sets the rim after the other faces' post hooks
 #pragma unroll
             for (int n = 0; n < 3; ++n) st4<NT>(V1 + n * cs + p, v[n]);
@@ -2065,27 +2065,6 @@ __global__ void k_tick(unsigned* __restrict__ numts)
 }
 
 // ---------------------------------------------------------------------------
-// soft / hard source application (Engine_Ext_Excitation::Apply2Voltages /
-// Apply2Current, engine_ext_excitation.cpp:33-99).  One thread per (component,
-// cell) group adds that cell's entries in list order, as the reference's
-// sequential loop does.  numTS is read from the device counter; the
-// current-side source runs after the counter advanced, hence ts_bias = -1.
-// ---------------------------------------------------------------------------
-__global__ void k_excite(float* __restrict__ F, unsigned G, const unsigned* __restrict__ gbeg,
-                         const unsigned long long* __restrict__ glin, const float* __restrict__ amp,
-                         const unsigned* __restrict__ delay, const float* __restrict__ sig, unsigned length,
-                         int period, const unsigned* __restrict__ numts, int ts_bias)
-{
-    const unsigned g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= G) return;
-    const int ts = (int)*numts + ts_bias;
-    const unsigned long long i = glin[g];
-    float v = F[i];
-    for (unsigned k = gbeg[g]; k < gbeg[g + 1]; ++k) v = v + amp[k] * sig[exc_sample(ts, delay[k], period, length)];
-    F[i] = v;
-}
-
-// ---------------------------------------------------------------------------
 // Mur ABC (Engine_Ext_Mur_ABC, engine_ext_mur_abc.cpp:68-178)
 // ---------------------------------------------------------------------------
 struct MurDev {
@@ -2099,46 +2078,6 @@ struct MurDev {
     float* mPP;
     unsigned start_ts;
 };
-
-__global__ void k_mur_pre(float* __restrict__ V, const MurDev m, const unsigned* __restrict__ numts)
-{
-    const unsigned k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= m.na * m.nb || *numts < m.start_ts) return;
-    const unsigned f = m.face[k], s = m.shift[k];
-    m.mP[k] = V[m.offP + s] - m.cP[k] * V[m.offP + f];
-    m.mPP[k] = V[m.offPP + s] - m.cPP[k] * V[m.offPP + f];
-}
-
-__global__ void k_mur_post(const float* __restrict__ V, const MurDev m, const unsigned* __restrict__ numts)
-{
-    const unsigned k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= m.na * m.nb || *numts < m.start_ts) return;
-    const unsigned s = m.shift[k];
-    m.mP[k] = m.mP[k] + m.cP[k] * V[m.offP + s];
-    m.mPP[k] = m.mPP[k] + m.cPP[k] * V[m.offPP + s];
-}
-
-__global__ void k_mur_apply(float* __restrict__ V, const MurDev m, const unsigned* __restrict__ numts)
-{
-    const unsigned k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= m.na * m.nb || *numts < m.start_ts) return;
-    const unsigned f = m.face[k];
-    V[m.offP + f] = m.mP[k];
-    V[m.offPP + f] = m.mPP[k];
-}
-
-// k_mur_apply at the listed points only (the rim of a face whose other
-// points the tiled quad sweep sets)
-__global__ void k_mur_apply_rim(float* __restrict__ V, const MurDev m, const unsigned* __restrict__ rim, unsigned n,
-                                const unsigned* __restrict__ numts)
-{
-    const unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n || *numts < m.start_ts) return;
-    const unsigned k = rim[t];
-    const unsigned f = m.face[k];
-    V[m.offP + f] = m.mP[k];
-    V[m.offPP + f] = m.mPP[k];
-}
 
 // The current update (curr_tile's arithmetic, FDTD/engine.cpp:170-222) redone
 // from the final voltages V1 and the currents of state n, into I1, for the
@@ -2223,32 +2162,6 @@ struct RlcDev {
 
 __device__ __forceinline__ unsigned rlc_slot(unsigned ts, unsigned i) { return (2u * ((ts + 1u) % 3u) + i) % 3u; }
 
-__global__ void k_rlc_pre(const RlcDev r, const unsigned* __restrict__ numts)
-{
-    const unsigned k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= r.count) return;
-    const unsigned ts = *numts;
-    const float* Vd1 = r.vd + rlc_slot(ts, 1) * r.count;
-    r.il[k] = r.il[k] + (r.c[0][k] * r.c[1][k]) * Vd1[k];
-}
-
-__global__ void k_rlc_apply(float* __restrict__ V, const RlcDev r, const unsigned* __restrict__ numts)
-{
-    const unsigned k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= r.count) return;
-    const unsigned ts = *numts;
-    float* V0 = r.vd + rlc_slot(ts, 0) * r.count;
-    const float* V2 = r.vd + rlc_slot(ts, 2) * r.count;
-    float* J0 = r.jn + rlc_slot(ts, 0) * r.count;
-    const float* J1 = r.jn + rlc_slot(ts, 1) * r.count;
-    const float* J2 = r.jn + rlc_slot(ts, 2) * r.count;
-    float v = V[r.lin[k]];
-    v = r.c[2][k] * (v - r.il[k] + r.c[3][k] * V2[k] + r.c[4][k] * J1[k] + r.c[5][k] * J2[k]);
-    V0[k] = v;
-    J0[k] = r.c[6][k] * (v - V2[k]) - (r.c[7][k] * r.c[6][k]) * J1[k] - (r.c[8][k] * r.c[6][k]) * J2[k];
-    V[r.lin[k]] = v;
-}
-
 // ---------------------------------------------------------------------------
 // Lorentz / Drude ADE (engine_ext_lorentzmaterial.cpp:79-173,
 // engine_ext_dispersive.cpp:76-132)
@@ -2263,33 +2176,208 @@ struct LorDev {
     float* lor;            // [3][count]
 };
 
-__global__ void k_lor_pre(const float* __restrict__ F, unsigned long long cs, const LorDev d)
+// one term of the ADE current subtracted from a cell's component
+struct LorTerm {
+    const float* ade;              // the order's [3][count]
+    unsigned k, count;
+};
+
+// steady-state detection (k_ss_eval)
+struct SteadyDev {
+    unsigned n, p, cap;
+    const unsigned long long* lin;   // [n] component * cs + cell
+    float* rec;                      // [n][2p]
+    double* state;                   // [0] last max diff, [1] last total energy, [2] evaluations
+    unsigned* hist_ts;               // [cap]
+    double* hist_diff;               // [cap]
+};
+
+// ---------------------------------------------------------------------------
+// Extension hooks around the two half steps (FDTD/engine.cpp:224-265).  Each
+// hook touches a face or a cell list, microseconds of work, so a step of an
+// engine with several extensions is bound by its launches (a small kernel in
+// a replayed graph costs 2.5-4.5 us from start to start, whatever it does).
+// One launch therefore runs every hook that may run concurrently: the host
+// (setup_hooks) keeps the reference's order and opens a new launch only where
+// a hook reads or writes a field element that an earlier hook of the launch
+// writes.  A workgroup belongs to one job (first[] in the kernel arguments).
+// Six Mur faces with steady-state detection (96 x 90 x 70): 22 -> 6 launches
+// and 66.0 -> 32.4 us per step; Drude, Lorentz and Debye boxes with RLC
+// elements (72^3): 17 -> 6 launches and 38.3 -> 23.0 us per step; one Mur
+// face (27 x 11 x 33): 6 -> 4 launches and 17.4 -> 15.3 us per step; 512 x
+// 384 x 320 layers around the quad sweep: 0.984 -> 0.959 ms per step.
+//
+//   MurPre / MurPost / MurApply  Engine_Ext_Mur_ABC (engine_ext_mur_abc.cpp:68-178);
+//                  the faces' applies run in reverse creation order, so where
+//                  two faces set one element the face created first wins:
+//                  over[] marks, per point and component, the earlier faces
+//                  (bit = creation index) that set the element too.
+//                  MurPostApply: post and apply of a face in one job, where no
+//                  face's apply sets what a post reads
+//   RlcPre / RlcApply  Engine_Ext_LumpedRLC (engine_ext_lumpedRLC.cpp:83-147)
+//   LorPre / LorApply  Engine_Ext_LorentzMaterial (engine_ext_lorentzmaterial.cpp:79-173,
+//                  engine_ext_dispersive.cpp:76-132); the orders' terms of a
+//                  cell are subtracted one after another in creation order
+//   Excite         Engine_Ext_Excitation (engine_ext_excitation.cpp:33-99): one
+//                  thread per (component, cell) group adds its entries in
+//                  list order; the current side of the two half steps runs
+//                  after the counter advanced (ts_bias -1)
+//   SteadyRecord   Engine_Ext_SteadyState's record (engine_ext_steadystate.cpp:50-64)
+// ---------------------------------------------------------------------------
+enum HookKind { kMurPre, kMurPost, kMurPostApply, kMurApply, kRlcPre, kRlcApply, kLorPre, kLorApply, kExcite, kSteadyRecord };
+
+constexpr unsigned kMaxHookJobs = 12;   // jobs of one launch
+constexpr unsigned kMurMaskFaces = 8;   // faces that over[] can name
+
+struct HookJob {
+    int kind;
+    int curr;                      // the field it works on: 0 voltages, 1 currents
+    unsigned n;                    // threads
+    MurDev mur;
+    const unsigned* list;          // MurApply: the points (null: all)
+    const unsigned char* over[2];  // MurApply: earlier faces setting the element (null: none)
+    unsigned start[kMurMaskFaces]; // MurApply: first timestep of each face
+    RlcDev rlc;
+    LorDev lor;
+    const unsigned* cell;          // LorApply: cells, their term ranges and terms
+    const unsigned* beg;
+    const LorTerm* term;
+    const unsigned* gbeg;          // Excite
+    const unsigned long long* glin;
+    const float* amp;
+    const unsigned* delay;
+    const float* sig;
+    unsigned length;
+    int period, ts_bias;
+    SteadyDev ss;
+};
+
+struct HookLaunch {
+    const HookJob* jobs;           // device memory
+    unsigned n;
+    unsigned first[kMaxHookJobs];  // first workgroup of each job
+    unsigned nblk;
+};
+
+__device__ __forceinline__ bool mur_overset(const HookJob& J, int c, unsigned k, unsigned ts)
 {
-    const unsigned k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= d.count) return;
+    if (!J.over[c]) return false;
+    const unsigned m = J.over[c][k];
+    bool o = false;
 #pragma unroll
-    for (int n = 0; n < 3; ++n) {
-        const unsigned j = n * d.count + k;
-        const float f = F[n * cs + d.lin[k]];
-        if (d.clor) {
-            d.lor[j] = d.lor[j] + d.clor[j] * d.ade[j];
-            float a = d.ade[j] * d.cint[j];
-            d.ade[j] = a + d.cext[j] * (f - d.lor[j]);
-        } else {
-            float a = d.ade[j] * d.cint[j];
-            d.ade[j] = a + d.cext[j] * f;
-        }
-    }
+    for (unsigned j = 0; j < kMurMaskFaces; ++j) o = o || ((m >> j & 1u) && ts >= J.start[j]);
+    return o;
 }
 
-__global__ void k_lor_apply(float* __restrict__ F, unsigned long long cs, const LorDev d)
+__global__ __launch_bounds__(kBlock) void k_hooks(float* __restrict__ V, float* __restrict__ I,
+                                                  const unsigned long long cs, const HookLaunch L,
+                                                  const unsigned* __restrict__ numts)
 {
-    const unsigned k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= d.count) return;
+    unsigned w = 0, f = 0;
 #pragma unroll
-    for (int n = 0; n < 3; ++n) {
-        const unsigned long long i = n * cs + d.lin[k];
-        F[i] = F[i] - d.ade[n * d.count + k];
+    for (unsigned i = 1; i < kMaxHookJobs; ++i)
+        if (i < L.n && blockIdx.x >= L.first[i]) {
+            w = i;
+            f = L.first[i];
+        }
+    const HookJob& J = L.jobs[w];
+    unsigned k = (blockIdx.x - f) * kBlock + threadIdx.x;
+    if (k >= J.n) return;
+    const unsigned ts = *numts;
+    float* F = J.curr ? I : V;
+    switch (J.kind) {
+    case kMurPre: {
+        const MurDev& m = J.mur;
+        if (ts < m.start_ts) return;
+        const unsigned p = m.face[k], s = m.shift[k];
+        m.mP[k] = F[m.offP + s] - m.cP[k] * F[m.offP + p];
+        m.mPP[k] = F[m.offPP + s] - m.cPP[k] * F[m.offPP + p];
+        return;
+    }
+    case kMurPost:
+    case kMurPostApply: {
+        const MurDev& m = J.mur;
+        if (ts < m.start_ts) return;
+        const unsigned s = m.shift[k];
+        const float a = m.mP[k] + m.cP[k] * F[m.offP + s];
+        const float b = m.mPP[k] + m.cPP[k] * F[m.offPP + s];
+        if (J.kind == kMurPost) {
+            m.mP[k] = a;
+            m.mPP[k] = b;
+            return;
+        }
+        const unsigned p = m.face[k];
+        F[m.offP + p] = a;
+        F[m.offPP + p] = b;
+        return;
+    }
+    case kMurApply: {
+        const MurDev& m = J.mur;
+        if (ts < m.start_ts) return;
+        if (J.list) k = J.list[k];
+        const unsigned p = m.face[k];
+        if (!mur_overset(J, 0, k, ts)) F[m.offP + p] = m.mP[k];
+        if (!mur_overset(J, 1, k, ts)) F[m.offPP + p] = m.mPP[k];
+        return;
+    }
+    case kRlcPre: {
+        const RlcDev& r = J.rlc;
+        const float* Vd1 = r.vd + rlc_slot(ts, 1) * r.count;
+        r.il[k] = r.il[k] + (r.c[0][k] * r.c[1][k]) * Vd1[k];
+        return;
+    }
+    case kRlcApply: {
+        const RlcDev& r = J.rlc;
+        float* V0 = r.vd + rlc_slot(ts, 0) * r.count;
+        const float* V2 = r.vd + rlc_slot(ts, 2) * r.count;
+        float* J0 = r.jn + rlc_slot(ts, 0) * r.count;
+        const float* J1 = r.jn + rlc_slot(ts, 1) * r.count;
+        const float* J2 = r.jn + rlc_slot(ts, 2) * r.count;
+        float v = F[r.lin[k]];
+        v = r.c[2][k] * (v - r.il[k] + r.c[3][k] * V2[k] + r.c[4][k] * J1[k] + r.c[5][k] * J2[k]);
+        V0[k] = v;
+        J0[k] = r.c[6][k] * (v - V2[k]) - (r.c[7][k] * r.c[6][k]) * J1[k] - (r.c[8][k] * r.c[6][k]) * J2[k];
+        F[r.lin[k]] = v;
+        return;
+    }
+    case kLorPre: {                // k = component * count + cell
+        const LorDev& d = J.lor;
+        const unsigned n = k / d.count;
+        const float x = F[n * cs + d.lin[k - n * d.count]];
+        const float ade = d.ade[k] * d.cint[k];
+        if (d.clor) {
+            const float l = d.lor[k] + d.clor[k] * d.ade[k];
+            d.lor[k] = l;
+            d.ade[k] = ade + d.cext[k] * (x - l);
+        } else {
+            d.ade[k] = ade + d.cext[k] * x;
+        }
+        return;
+    }
+    case kLorApply: {              // k = component * cells + cell
+        const unsigned nc = J.n / 3u, n = k / nc, c = k - n * nc;
+        const unsigned long long i = n * cs + J.cell[c];
+        float x = F[i];
+        for (unsigned e = J.beg[c]; e < J.beg[c + 1]; ++e) {
+            const LorTerm T = J.term[e];
+            x = x - T.ade[n * T.count + T.k];
+        }
+        F[i] = x;
+        return;
+    }
+    case kExcite: {
+        const unsigned long long i = J.glin[k];
+        float v = F[i];
+        for (unsigned e = J.gbeg[k]; e < J.gbeg[k + 1]; ++e)
+            v = v + J.amp[e] * J.sig[exc_sample((int)ts + J.ts_bias, J.delay[e], J.period, J.length)];
+        F[i] = v;
+        return;
+    }
+    case kSteadyRecord: {
+        const SteadyDev& s = J.ss;
+        s.rec[(size_t)k * 2 * s.p + ts % (2 * s.p)] = F[s.lin[k]];
+        return;
+    }
     }
 }
 
@@ -2920,23 +3008,6 @@ __global__ void k_adj_src(float* __restrict__ lV, const AdjProbe* __restrict__ p
 // update.  Every step records the probe voltages at TS % 2p; at TS % p == 0,
 // TS >= 2p it compares the last two periods and the energy change.
 // ---------------------------------------------------------------------------
-struct SteadyDev {
-    unsigned n, p, cap;
-    const unsigned long long* lin;   // [n] component * cs + cell
-    float* rec;                      // [n][2p]
-    double* state;                   // [0] last max diff, [1] last total energy, [2] evaluations
-    unsigned* hist_ts;               // [cap]
-    double* hist_diff;               // [cap]
-};
-
-__global__ void k_ss_record(const float* __restrict__ V, const SteadyDev s, const unsigned* __restrict__ numts)
-{
-    const unsigned k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= s.n) return;
-    const unsigned rel = *numts % (2 * s.p);
-    s.rec[(size_t)k * 2 * s.p + rel] = V[s.lin[k]];
-}
-
 // one thread: the reference's evaluation, energy from k_energy's partials
 __global__ void k_ss_eval(const SteadyDev s, const double* __restrict__ part, unsigned nb,
                           const unsigned* __restrict__ numts)
@@ -3071,7 +3142,7 @@ struct ems_engine {
     unsigned qblk_all = 0, qblk_in = 0, qblk_out = 0;
     QBox* qbox_dev = nullptr;             // the three box lists, kMaxQBoxes each
     // voltage sources added by k_volt4 / k_volt (per-quad or per-column lists;
-    // beg null: k_excite adds them)
+    // beg null: the Excite hook adds them)
     ExcArgs qsrc{};
     bool qsplit = false;
     unsigned ntx = 0, nty = 0, fzdepth = 0, fnzc = 0;
@@ -3108,7 +3179,16 @@ struct ems_engine {
     // lumped RLC and dispersive lists
     std::vector<RlcDev> rlc;
     std::vector<LorDev> lor;
+    // their field elements and cells, and the steady-state probes' elements
+    std::vector<std::vector<unsigned long long>> h_rlc;
+    std::vector<std::vector<unsigned>> h_lor;
+    std::vector<unsigned long long> h_ss;
     std::vector<int> lor_v, lor_i;
+    // the extension hooks' launches (setup_hooks): before the voltage update,
+    // after it (the steady-state evaluation follows launch hooks_ss), after
+    // the current update
+    std::vector<HookLaunch> hooks_pre, hooks_v, hooks_i;
+    int hooks_ss = -1;
 
     // probes
     std::vector<ProbeDev> probes;
@@ -3444,7 +3524,7 @@ int ems_get_layout(const ems_engine* h, int* layout, unsigned* n_unique, int* pm
 }  // extern "C"
 
 // entries (list order) grouped per (component, cell) in order of first
-// appearance, as k_excite applies them, uploaded into E (device lists only)
+// appearance, as the Excite hook applies them, uploaded into E (device lists only)
 static int upload_exc_groups(ems_engine* h, const std::vector<ExcEnt>& ent, ems_engine::Exc& E)
 {
     const unsigned K = (unsigned)ent.size();
@@ -3476,6 +3556,7 @@ static int upload_exc_groups(ems_engine* h, const std::vector<ExcEnt>& ent, ems_
         gd[k] = ent[order[k]].delay;
     }
     E.G = G;
+    E.h_glin = glin;
     int rc;
     if ((rc = upload(h, &E.gbeg, gbeg.data(), G + 1)) || (rc = upload(h, &E.glin, glin.data(), G)) ||
         (rc = upload(h, &E.amp, ga.data(), K)) || (rc = upload(h, &E.delay, gd.data(), K)))
@@ -3779,6 +3860,7 @@ int ems_add_lumped_rlc(ems_engine* h, unsigned count, const unsigned* pos, const
     HIPCHK(hipMemset(r.jn, 0, 3 * count * sizeof(float)));
     HIPCHK(hipMemset(r.il, 0, count * sizeof(float)));
     h->rlc.push_back(r);
+    h->h_rlc.push_back(std::move(lin));
     return 0;
 }
 
@@ -3822,6 +3904,7 @@ int ems_add_lorentz(ems_engine* h, unsigned count, const unsigned* pos, const fl
         h->lor.push_back(d);
         (side ? h->lor_i : h->lor_v).push_back(on ? 1 : 0);
     }
+    h->h_lor.push_back(std::move(lin));
     return 0;
 }
 
@@ -4108,6 +4191,7 @@ int ems_set_steady_state(ems_engine* h, unsigned period_steps, unsigned nprobe, 
     const double st[3] = {1.0, 0.0, 0.0};
     HIPCHK(hipMemcpy(S.state, st, sizeof(st), hipMemcpyHostToDevice));
     h->ss = S;
+    h->h_ss = std::move(lin);
     h->has_ss = true;
     return 0;
 }
@@ -4295,6 +4379,308 @@ static int setup_vsrc(ems_engine* h)
     return 0;
 }
 
+}  // extern "C"
+
+// ---------------------------------------------------------------------------
+// Hook launches (k_hooks): the jobs of a phase in the reference's order, each
+// put into the phase's last launch unless it touches a field element that a
+// job of that launch sets, or sets one that a job of that launch touches.
+// ---------------------------------------------------------------------------
+namespace {
+
+struct HookPlan {
+    HookJob d{};
+    std::vector<unsigned long long> cells;    // sorted component * cs + cell of a list job
+    bool writes = true;                       // it sets field elements
+    const ems_engine::MurGeo* mur = nullptr;  // a Mur face's job
+    int face = -1;
+};
+
+// element e on the lines a Mur job reads (its neighbour line, before or
+// after the update) or sets (its face line)
+bool mur_touches(const ems_engine* h, const HookPlan& m, unsigned long long e, bool want_write)
+{
+    const int c = (int)(e / h->cs);
+    if (c == m.mur->ny) return false;
+    const unsigned long long p = e % h->cs;
+    const unsigned x[3] = {(unsigned)(p % h->N[0]), (unsigned)(p / h->N[0] % h->N[1]), (unsigned)(p / h->g.plane)};
+    const unsigned v = x[m.mur->ny];
+    const bool reads = m.d.kind != kMurApply && v == m.mur->shift;
+    const bool sets = m.d.kind != kMurPost && v == m.mur->line;
+    return want_write ? sets : reads || sets;
+}
+
+bool hooks_conflict(const ems_engine* h, const HookPlan& a, const HookPlan& b)
+{
+    if (a.mur && b.mur) {
+        if (a.face == b.face) return true;               // through the face's own values
+        auto hit = [&](const HookPlan& r, const HookPlan& w) {      // w's apply sets what r's post reads
+            if (w.d.kind == kMurPost || r.d.kind == kMurApply) return false;
+            return r.mur->ny != w.mur->ny || r.mur->shift == w.mur->line;
+        };
+        if (hit(a, b) || hit(b, a)) return true;
+        if (a.d.kind == kMurPost || b.d.kind == kMurPost) return false;
+        // two applies setting one element: over[] resolves them
+        return (a.mur->ny != b.mur->ny || a.mur->line == b.mur->line) && h->mur.size() > kMurMaskFaces;
+    }
+    if (a.mur || b.mur) {
+        const HookPlan& m = a.mur ? a : b;
+        const HookPlan& l = a.mur ? b : a;
+        for (unsigned long long e : l.cells)
+            if (mur_touches(h, m, e, !l.writes)) return true;
+        return false;
+    }
+    if (!a.writes && !b.writes) return false;
+    for (size_t i = 0, j = 0; i < a.cells.size() && j < b.cells.size();) {
+        if (a.cells[i] == b.cells[j]) return true;
+        if (a.cells[i] < b.cells[j]) ++i;
+        else ++j;
+    }
+    return false;
+}
+
+}  // namespace
+
+// the jobs as launches; `alone` ends a launch after job `alone` (its launch's
+// index goes to *at)
+static int build_hook_launches(ems_engine* h, const std::vector<HookPlan>& jobs, bool independent,
+                               std::vector<HookLaunch>& out, int alone = -1, int* at = nullptr)
+{
+    out.clear();
+    std::vector<std::vector<const HookPlan*>> sets;
+    bool closed = true;
+    for (size_t j = 0; j < jobs.size(); ++j) {
+        if (!jobs[j].d.n) continue;
+        bool fresh = closed || sets.back().size() >= kMaxHookJobs;
+        for (size_t i = 0; !fresh && !independent && i < sets.back().size(); ++i)
+            fresh = hooks_conflict(h, *sets.back()[i], jobs[j]);
+        if (fresh) sets.emplace_back();
+        sets.back().push_back(&jobs[j]);
+        closed = (int)j == alone;
+        if (closed && at) *at = (int)sets.size() - 1;
+    }
+    for (const auto& set : sets) {
+        HookLaunch L{};
+        std::vector<HookJob> d;
+        for (const HookPlan* q : set) {
+            L.first[L.n++] = L.nblk;
+            L.nblk += (q->d.n + kBlock - 1) / kBlock;
+            d.push_back(q->d);
+        }
+        HookJob* dj;
+        int rc = upload(h, &dj, d.data(), d.size());
+        if (rc) return rc;
+        L.jobs = dj;
+        out.push_back(L);
+    }
+    return 0;
+}
+
+// earlier faces (bit: creation index) that set the P (c = 0) or PP component
+// of each of face k's points too; null where there is none
+static int mur_over(ems_engine* h, int k, int c, const unsigned char** out)
+{
+    *out = nullptr;
+    if (h->mur.size() > kMurMaskFaces) return 0;
+    const auto& G = h->mur_geo[k];
+    const int nP = (G.ny + 1) % 3, nPP = (G.ny + 2) % 3, comp = c ? nPP : nP;
+    const MurDev& m = h->mur[k];
+    const bool tr = nP < nPP;             // device order of the points (ems_add_mur)
+    std::vector<unsigned char> over((size_t)m.na * m.nb, 0);
+    bool any = false;
+    for (int j = 0; j < k; ++j) {
+        const auto& J = h->mur_geo[j];
+        if (J.ny == comp || (J.ny == G.ny && J.line != G.line)) continue;
+        for (unsigned a = 0; a < m.na; ++a)
+            for (unsigned b = 0; b < m.nb; ++b) {
+                if (J.ny != G.ny && (J.ny == nP ? a : b) != J.line) continue;
+                over[tr ? (size_t)b * m.na + a : (size_t)a * m.nb + b] |= (unsigned char)(1u << j);
+                any = true;
+            }
+    }
+    if (!any) return 0;
+    unsigned char* d;
+    int rc = upload(h, &d, over.data(), over.size());
+    *out = d;
+    return rc;
+}
+
+static int setup_hooks(ems_engine* h)
+{
+    auto mur_job = [&](int kind, int k) {
+        HookPlan q;
+        q.d.kind = kind;
+        q.d.mur = h->mur[k];
+        q.d.n = h->mur[k].na * h->mur[k].nb;
+        q.mur = &h->mur_geo[k];
+        q.face = k;
+        return q;
+    };
+    auto exc_job = [&](const ems_engine::Exc& e, int curr, int bias) {
+        HookPlan q;
+        q.d.kind = kExcite;
+        q.d.curr = curr;
+        q.d.n = e.G;
+        q.d.gbeg = e.gbeg;
+        q.d.glin = e.glin;
+        q.d.amp = e.amp;
+        q.d.delay = e.delay;
+        q.d.sig = h->sig[curr];
+        q.d.length = h->sigLen;
+        q.d.period = h->period;
+        q.d.ts_bias = bias;
+        q.cells = e.h_glin;
+        std::sort(q.cells.begin(), q.cells.end());
+        return q;
+    };
+    const int nmur = (int)h->mur.size();
+    auto folded = [&](int k) { return k == h->mur_fold[0] || k == h->mur_fold[1]; };
+    auto mur_apply = [&](int k, HookPlan& q) {
+        q = mur_job(kMurApply, k);
+        for (int j = 0; j < nmur && j < (int)kMurMaskFaces; ++j) q.d.start[j] = h->mur[j].start_ts;
+        int rc = mur_over(h, k, 0, &q.d.over[0]);
+        return rc ? rc : mur_over(h, k, 1, &q.d.over[1]);
+    };
+    int rc;
+    std::vector<HookPlan> pre, v, c;
+    // before the voltage update: nothing here sets a field element, and the
+    // current side's ADE reads currents that no hook sets before the current update
+    for (int k = 0; k < nmur; ++k)
+        if (!folded(k)) pre.push_back(mur_job(kMurPre, k));
+    for (int side = 0; side < 2; ++side)
+        for (size_t k = side; k < h->lor.size(); k += 2) {
+            if (!(side ? h->lor_i : h->lor_v)[k / 2]) continue;
+            HookPlan q;
+            q.d.kind = kLorPre;
+            q.d.curr = side;
+            q.d.n = 3 * h->lor[k].count;
+            q.d.lor = h->lor[k];
+            pre.push_back(q);
+        }
+    for (const auto& r : h->rlc) {
+        HookPlan q;
+        q.d.kind = kRlcPre;
+        q.d.n = r.count;
+        q.d.rlc = r;
+        pre.push_back(q);
+    }
+    if ((rc = build_hook_launches(h, pre, true, h->hooks_pre))) return rc;
+    if (h->fused) {
+        // around the quad sweep: posts, applies (the rims of the faces inside
+        // the sweep), then the deferred sources; nothing else has a form there
+        if (!nmur) return 0;
+        for (int k = nmur - 1; k >= 0; --k)
+            if (!folded(k)) v.push_back(mur_job(kMurPost, k));
+        for (int k = nmur - 1; k >= 0; --k) {
+            HookPlan q;
+            if ((rc = mur_apply(k, q))) return rc;
+            const int side = k == h->mur_fold[0] ? 0 : k == h->mur_fold[1] ? 1 : -1;
+            if (side >= 0) {
+                q.d.list = h->mur_rim[side];
+                q.d.n = h->nrim[side];
+            }
+            v.push_back(q);
+        }
+        if (h->exc_def[0].G) v.push_back(exc_job(h->exc_def[0], 0, 0));
+        if ((rc = build_hook_launches(h, v, false, h->hooks_v))) return rc;
+        if (h->exc_def[1].G) c.push_back(exc_job(h->exc_def[1], 1, 0));
+        return build_hook_launches(h, c, false, h->hooks_i);
+    }
+    // after the voltage update: Mur post (reverse creation order, reads only),
+    // steady-state record, lumped RLC, Lorentz, Mur apply (reverse creation
+    // order), excitation
+    std::vector<HookPlan> list;               // RLC and Lorentz, in order
+    for (size_t k = 0; k < h->rlc.size(); ++k) {
+        HookPlan q;
+        q.d.kind = kRlcApply;
+        q.d.n = h->rlc[k].count;
+        q.d.rlc = h->rlc[k];
+        q.cells = h->h_rlc[k];
+        std::sort(q.cells.begin(), q.cells.end());
+        list.push_back(q);
+    }
+    auto lor_apply = [&](int side, HookPlan& q) {
+        // a cell's orders in creation order
+        std::vector<std::pair<unsigned, LorTerm>> t;
+        for (size_t k = side; k < h->lor.size(); k += 2) {
+            if (!(side ? h->lor_i : h->lor_v)[k / 2]) continue;
+            const LorDev& d = h->lor[k];
+            for (unsigned j = 0; j < d.count; ++j) t.push_back({h->h_lor[k / 2][j], LorTerm{d.ade, j, d.count}});
+        }
+        std::stable_sort(t.begin(), t.end(), [](const auto& l, const auto& r) { return l.first < r.first; });
+        std::vector<unsigned> cell, beg;
+        std::vector<LorTerm> term;
+        for (const auto& e : t) {
+            if (cell.empty() || cell.back() != e.first) {
+                cell.push_back(e.first);
+                beg.push_back((unsigned)term.size());
+            }
+            term.push_back(e.second);
+        }
+        beg.push_back((unsigned)term.size());
+        q.d.kind = kLorApply;
+        q.d.curr = side;
+        q.d.n = 3 * (unsigned)cell.size();
+        if (!q.d.n) return 0;
+        for (int n = 0; n < 3; ++n)
+            for (unsigned x : cell) q.cells.push_back(n * h->cs + x);
+        unsigned *dc, *db;
+        LorTerm* dt;
+        int r;
+        if ((r = upload(h, &dc, cell.data(), cell.size())) || (r = upload(h, &db, beg.data(), beg.size())) ||
+            (r = upload(h, &dt, term.data(), term.size())))
+            return r;
+        q.d.cell = dc;
+        q.d.beg = db;
+        q.d.term = dt;
+        return 0;
+    };
+    HookPlan lv, li;
+    if ((rc = lor_apply(0, lv)) || (rc = lor_apply(1, li))) return rc;
+    if (lv.d.n) list.push_back(lv);
+    std::vector<HookPlan> post, apply;
+    for (int k = nmur - 1; k >= 0; --k) {
+        post.push_back(mur_job(kMurPost, k));
+        HookPlan q;
+        if ((rc = mur_apply(k, q))) return rc;
+        apply.push_back(q);
+    }
+    // post and apply as one job where that changes no value read
+    bool joint = nmur > 0;
+    for (int a = 0; a < nmur && joint; ++a) {
+        for (int b = 0; b < nmur && joint; ++b)
+            joint = h->mur_geo[a].ny == h->mur_geo[b].ny && h->mur_geo[a].shift != h->mur_geo[b].line &&
+                    (a == b || h->mur_geo[a].line != h->mur_geo[b].line);
+        for (const auto& q : list) joint = joint && !hooks_conflict(h, post[a], q);
+    }
+    if (joint)
+        for (auto& q : apply) q.d.kind = kMurPostApply;
+    else
+        v = post;
+    int ss = -1;
+    if (h->has_ss) {
+        HookPlan q;
+        q.d.kind = kSteadyRecord;
+        q.d.n = h->ss.n;
+        q.d.ss = h->ss;
+        q.writes = false;
+        q.cells = h->h_ss;
+        std::sort(q.cells.begin(), q.cells.end());
+        ss = (int)v.size();
+        v.push_back(q);
+    }
+    v.insert(v.end(), list.begin(), list.end());
+    v.insert(v.end(), apply.begin(), apply.end());
+    if (h->exc[0].G && !h->qsrc.beg) v.push_back(exc_job(h->exc[0], 0, 0));
+    // the steady-state evaluation's energy reads the voltages before any hook sets them
+    if ((rc = build_hook_launches(h, v, false, h->hooks_v, ss, &h->hooks_ss))) return rc;
+    if (li.d.n) c.push_back(li);
+    if (h->exc[1].G) c.push_back(exc_job(h->exc[1], 1, -1));
+    return build_hook_launches(h, c, false, h->hooks_i);
+}
+
+extern "C" {
+
 int ems_set_quad(ems_engine* h, int mode)
 {
     if (!h) return fail(EMS_E_ARG, "null handle");
@@ -4322,6 +4708,7 @@ int ems_init(ems_engine* h)
     if ((rc = setup_fused(h))) return rc;
     if ((rc = setup_quad(h))) return rc;
     if ((rc = setup_vsrc(h))) return rc;
+    if ((rc = setup_hooks(h))) return rc;
     // small compressed tables (both half steps' within 32 KiB) go to LDS in the quad kernels
     h->lds_tab = h->cmp && (size_t)4 * h->n_unique * sizeof(float4) <= kLdsTabBytes;
     if (const char* lt = std::getenv("EMS_LDS_TAB")) h->lds_tab = h->lds_tab && std::atoi(lt) != 0;
@@ -4754,17 +5141,23 @@ void quad_step(ems_engine* h)
     else launch_step4_t<false>(h, a, nblk);
 }
 
+void launch_hook(ems_engine* h, const HookLaunch& L, float* V, float* I)
+{
+    hipLaunchKernelGGL(k_hooks, dim3(L.nblk), dim3(kBlock), 0, h->stream, V, I, h->cs, L, h->numts_dev);
+}
+
+void launch_hooks(ems_engine* h, const std::vector<HookLaunch>& hooks, float* V, float* I)
+{
+    for (const auto& L : hooks) launch_hook(h, L, V, I);
+}
+
 // one fused step from state n (h->V, h->I, current fluxes) into the second
 // buffers, which then become the current state
 void fused_step(ems_engine* h, hipEvent_t* ev)
 {
     const unsigned T = 256;
     // Mur pre hooks read state n (FDTD/engine.cpp:224-265 order; only the quad sweep has Mur)
-    for (size_t k = 0; k < h->mur.size(); ++k) {
-        if ((int)k == h->mur_fold[0] || (int)k == h->mur_fold[1]) continue;     // in k_step4t
-        const auto& m = h->mur[k];
-        hipLaunchKernelGGL(k_mur_pre, dim3((m.na * m.nb + T - 1) / T), dim3(T), 0, h->stream, h->V, m, h->numts_dev);
-    }
+    launch_hooks(h, h->hooks_pre, h->V, h->I);
     if (ev) (void)hipEventRecord(ev[0], h->stream);
     if (h->fused == 3) quad_step(h);
     else if (h->fused == 2) column_step(h);
@@ -4777,28 +5170,7 @@ void fused_step(ems_engine* h, hipEvent_t* ev)
         // state n+1: Mur post (reverse creation order) on the swept voltages,
         // Mur apply, the deferred voltage sources, then the current update of
         // the planes next to each face again, with their current sources
-        for (int k = (int)h->mur.size() - 1; k >= 0; --k) {
-            if (k == h->mur_fold[0] || k == h->mur_fold[1]) continue;          // in k_step4t
-            const auto& m = h->mur[k];
-            hipLaunchKernelGGL(k_mur_post, dim3((m.na * m.nb + T - 1) / T), dim3(T), 0, h->stream, h->V_alt, m,
-                               h->numts_dev);
-        }
-        for (int k = (int)h->mur.size() - 1; k >= 0; --k) {
-            const auto& m = h->mur[k];
-            const int side = k == h->mur_fold[0] ? 0 : k == h->mur_fold[1] ? 1 : -1;
-            if (side >= 0) {
-                if (h->nrim[side])
-                    hipLaunchKernelGGL(k_mur_apply_rim, dim3((h->nrim[side] + T - 1) / T), dim3(T), 0, h->stream,
-                                       h->V_alt, m, h->mur_rim[side], h->nrim[side], h->numts_dev);
-                continue;
-            }
-            hipLaunchKernelGGL(k_mur_apply, dim3((m.na * m.nb + T - 1) / T), dim3(T), 0, h->stream, h->V_alt, m,
-                               h->numts_dev);
-        }
-        const auto& e0 = h->exc_def[0];
-        if (e0.G)
-            hipLaunchKernelGGL(k_excite, dim3((e0.G + T - 1) / T), dim3(T), 0, h->stream, h->V_alt, e0.G, e0.gbeg,
-                               e0.glin, e0.amp, e0.delay, h->sig[0], h->sigLen, h->period, h->numts_dev, 0);
+        launch_hooks(h, h->hooks_v, h->V_alt, h->I_alt);
         for (const auto& b : h->bands) {
             const unsigned long long cnt = (unsigned long long)(b.hi - b.lo + 1) * h->N[0] * h->N[1] * h->N[2] /
                                            h->N[b.axis];
@@ -4808,10 +5180,7 @@ void fused_step(ems_engine* h, hipEvent_t* ev)
         if (h->ncells)
             hipLaunchKernelGGL(k_curr_cells, dim3((h->ncells + T - 1) / T), dim3(T), 0, h->stream, h->g, h->V_alt,
                                h->I, h->I_alt, h->kI, h->cell_list, h->ncells);
-        const auto& e1 = h->exc_def[1];
-        if (e1.G)
-            hipLaunchKernelGGL(k_excite, dim3((e1.G + T - 1) / T), dim3(T), 0, h->stream, h->I_alt, e1.G, e1.gbeg,
-                               e1.glin, e1.amp, e1.delay, h->sig[1], h->sigLen, h->period, h->numts_dev, 0);
+        launch_hooks(h, h->hooks_i, h->V_alt, h->I_alt);
     }
     hipLaunchKernelGGL(k_tick, dim3(1), dim3(64), 0, h->stream, h->numts_dev);
     if (ev) (void)hipEventRecord(ev[3], h->stream);
@@ -4867,67 +5236,27 @@ static int launch_step(ems_engine* h, hipEvent_t* ev)
     }
     const GridDesc& g = h->g;
     const unsigned nblk = g.qtiles * g.nzc;
-    const unsigned T = 256;
-    // -- voltage pre hooks: Mur (creation order), Lorentz, lumped RLC; UPML pre is fused
-    for (size_t k = 0; k < h->mur.size(); ++k) {
-        if ((int)k == h->mur_fold[0] || (int)k == h->mur_fold[1]) continue;     // in k_step4t
-        const auto& m = h->mur[k];
-        hipLaunchKernelGGL(k_mur_pre, dim3((m.na * m.nb + T - 1) / T), dim3(T), 0, h->stream, h->V, m, h->numts_dev);
-    }
-    for (size_t k = 0; k < h->lor.size(); k += 2)
-        if (h->lor_v[k / 2])
-            hipLaunchKernelGGL(k_lor_pre, dim3((h->lor[k].count + T - 1) / T), dim3(T), 0, h->stream, h->V, h->cs, h->lor[k]);
-    for (const auto& r : h->rlc)
-        hipLaunchKernelGGL(k_rlc_pre, dim3((r.count + T - 1) / T), dim3(T), 0, h->stream, r, h->numts_dev);
+    // -- pre hooks: Mur, lumped RLC, Lorentz of both sides; UPML pre is fused
+    launch_hooks(h, h->hooks_pre, h->V, h->I);
     if (ev) (void)hipEventRecord(ev[0], h->stream);
     dispatch_update(h, false, nblk);
     if (ev) (void)hipEventRecord(ev[1], h->stream);
-    // -- post hooks: Mur (reverse creation order, all read-only on V)
-    for (int k = (int)h->mur.size() - 1; k >= 0; --k) {
-        const auto& m = h->mur[k];
-        hipLaunchKernelGGL(k_mur_post, dim3((m.na * m.nb + T - 1) / T), dim3(T), 0, h->stream, h->V, m, h->numts_dev);
-    }
-    // -- apply hooks: steady-state record (priority +2e6), lumped RLC, Lorentz,
-    //    Mur (reverse creation order), excitation
-    if (h->has_ss) {
-        const SteadyDev& S = h->ss;
-        hipLaunchKernelGGL(k_ss_record, dim3((S.n + T - 1) / T), dim3(T), 0, h->stream, h->V, S, h->numts_dev);
-        if (h->numTS % S.p == 0 && h->numTS >= 2 * S.p) {
+    // -- post and apply hooks: Mur post, steady-state record (priority +2e6),
+    //    lumped RLC, Lorentz, Mur apply, excitation
+    for (size_t k = 0; k < h->hooks_v.size(); ++k) {
+        launch_hook(h, h->hooks_v[k], h->V, h->I);
+        if ((int)k == h->hooks_ss && h->numTS % h->ss.p == 0 && h->numTS >= 2 * h->ss.p) {
             const unsigned nb = 1024;
             hipLaunchKernelGGL(k_energy, dim3(nb), dim3(kBlock), 0, h->stream, h->V, h->I, h->cs, h->N[0], h->N[1],
                                h->N[2], h->ss_part);
-            hipLaunchKernelGGL(k_ss_eval, dim3(1), dim3(64), 0, h->stream, S, h->ss_part, nb, h->numts_dev);
+            hipLaunchKernelGGL(k_ss_eval, dim3(1), dim3(64), 0, h->stream, h->ss, h->ss_part, nb, h->numts_dev);
         }
     }
-    for (const auto& r : h->rlc)
-        hipLaunchKernelGGL(k_rlc_apply, dim3((r.count + T - 1) / T), dim3(T), 0, h->stream, h->V, r, h->numts_dev);
-    for (size_t k = 0; k < h->lor.size(); k += 2)
-        if (h->lor_v[k / 2])
-            hipLaunchKernelGGL(k_lor_apply, dim3((h->lor[k].count + T - 1) / T), dim3(T), 0, h->stream, h->V, h->cs, h->lor[k]);
-    for (int k = (int)h->mur.size() - 1; k >= 0; --k) {
-        const auto& m = h->mur[k];
-        hipLaunchKernelGGL(k_mur_apply, dim3((m.na * m.nb + T - 1) / T), dim3(T), 0, h->stream, h->V, m, h->numts_dev);
-    }
-    if (h->exc[0].G && !h->qsrc.beg) {
-        const auto& e = h->exc[0];
-        hipLaunchKernelGGL(k_excite, dim3((e.G + T - 1) / T), dim3(T), 0, h->stream, h->V, e.G, e.gbeg, e.glin, e.amp,
-                           e.delay, h->sig[0], h->sigLen, h->period, h->numts_dev, 0);
-    }
-    // -- current half step: Lorentz pre, fused UPML + update, Lorentz apply, excitation
-    for (size_t k = 1; k < h->lor.size(); k += 2)
-        if (h->lor_i[k / 2])
-            hipLaunchKernelGGL(k_lor_pre, dim3((h->lor[k].count + T - 1) / T), dim3(T), 0, h->stream, h->I, h->cs, h->lor[k]);
+    // -- current half step: fused UPML + update, Lorentz apply, excitation
     if (ev) (void)hipEventRecord(ev[2], h->stream);
     dispatch_update(h, true, nblk);
     if (ev) (void)hipEventRecord(ev[3], h->stream);
-    for (size_t k = 1; k < h->lor.size(); k += 2)
-        if (h->lor_i[k / 2])
-            hipLaunchKernelGGL(k_lor_apply, dim3((h->lor[k].count + T - 1) / T), dim3(T), 0, h->stream, h->I, h->cs, h->lor[k]);
-    if (h->exc[1].G) {
-        const auto& e = h->exc[1];
-        hipLaunchKernelGGL(k_excite, dim3((e.G + T - 1) / T), dim3(T), 0, h->stream, h->I, e.G, e.gbeg, e.glin, e.amp,
-                           e.delay, h->sig[1], h->sigLen, h->period, h->numts_dev, -1);
-    }
+    launch_hooks(h, h->hooks_i, h->V, h->I);
     HIPCHK(hipGetLastError());
     return 0;
 }

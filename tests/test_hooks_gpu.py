@@ -1,0 +1,69 @@
+"""Extension hooks sharing a launch: every combination in which one hook reads
+or sets an element that another sets (Mur faces that meet at edges, a single
+axis of Mur faces, sources and ADE cells on face and neighbour lines, lumped
+elements in dispersive cells, steady-state probes on a face) against the
+oracle, bit for bit."""
+import numpy as np
+import pytest
+
+from oracle.operator_ref import RefOperator
+from oracle.oracle import RefEngine
+from openems_amd import scenes
+from openems_amd.engine import EngineHIP
+from openems_amd.operator import Operator
+from openems_amd.simulation import steady_state_probes
+from tests.test_engine_gpu import _oracle_ade
+
+pytestmark = pytest.mark.gpu
+
+
+def _layers(bc, at=None):
+    """Mur layers, the sheet source across every face line, or one on line `at` of x"""
+    s = dict(scenes.mur_layers(30, 26, 22, 120), bc=bc)
+    if at is not None:
+        lx, ly, lz = s["lines"]
+        s["excitations"] = [{"type": 0, "val": (0.0, 1.0, 0.5), "start": (lx[at], ly[8], lz[6]), "stop": (lx[at], ly[9], lz[7])}]
+    return s
+
+
+def _dispersive(bc):
+    """ADE cells and lumped elements beside and on Mur lines: the Drude box reaches to the x = 0 face"""
+    s = scenes.dispersive_rlc(36, 120)
+    L = s["lines"]
+    s["bc"] = bc
+    s["materials"][0]["start"] = (L[0][0], L[1][0], L[2][10])
+    s["lumped"][1]["start"] = (L[0][12], L[1][15], L[2][16])      # inside the Drude box: both set its elements
+    s["lumped"][1]["stop"] = (L[0][12], L[1][15], L[2][20])
+    s["materials"][0]["stop"] = (L[0][14], L[1][24], L[2][24])
+    return s
+
+
+CASES = [
+    ("mur_all", lambda: _layers([2] * 6), True),
+    ("mur_x_pair", lambda: _layers([2, 2, 0, 0, 0, 0], 15), False),
+    ("mur_x_pair_source_on_neighbour", lambda: _layers([2, 2, 0, 0, 0, 0], 1), True),
+    ("mur_x_low_source_on_face", lambda: _layers([2, 0, 1, 0, 0, 1], 0), False),
+    ("dispersive_pml", lambda: _dispersive([3] * 6), False),
+    ("dispersive_mur_all", lambda: _dispersive([2] * 6), False),
+    ("dispersive_mur_x", lambda: _dispersive([2, 2, 0, 0, 0, 0]), False),
+]
+
+
+@pytest.mark.parametrize("name,make,steady", CASES, ids=[c[0] for c in CASES])
+def test_hooks_match_oracle(gpu, name, make, steady):
+    scene = make()
+    print("case hooks", name, flush=True)
+    op = Operator(scene)
+    ss = steady_state_probes(op) if steady else None
+    eng = EngineHIP(op, fused=False, steady_state=ss)
+    eng.IterateTS(120)
+    ref = RefOperator(scene).build()
+    lor, rlc = _oracle_ade(ref) if scene.get("lumped") else ([], None)
+    e = RefEngine(ref, "basic", lorentz=lor, rlc=rlc) if lor else RefEngine(ref, "basic")
+    e.iterate(120)
+    rv, rc = e.raw_views()
+    assert np.max(np.abs(rv)) > 0
+    assert np.array_equal(eng.get_volt(), rv)
+    assert np.array_equal(eng.get_curr(), rc)
+    eng.close()
+    e.close()
