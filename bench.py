@@ -440,7 +440,8 @@ def run_plain_cavity(steps=2000, cpu=True, nthreads=1):
                        f"E point + voltage line probes, {steps} steps",
            "cells": int(cells), "value": round(cells * steps / wall / 1e6, 1), "unit": "MCells/s",
            "ms_per_step": round(wall * 1e3 / steps, 5),
-           "layout": f"{lay}, two half steps, {'four x cells per lane' if quad else 'one cell per lane'}, "
+           "layout": f"{lay}, " + ("two timesteps per launch, single steps as " if eng.pair()[0] else "")
+                     + f"two half steps, {'four x cells per lane' if quad else 'one cell per lane'}, "
                      f"timestep chunks replayed as HIP graphs",
            "note": "3.1 MB per field: cache-resident and launch-bound, no HBM roofline"}
     if cpu:
@@ -520,14 +521,21 @@ def main():
     play = play or "plain"
     fused, zdepth = eng.fused()
     quad, qzdepth = eng.quad()
-    if fused:
+    pair, ptile, _ = eng.pair()
+    if pair:
+        # two steps per launch: the fields and fluxes read and written once
+        bytes_per_launch = FUSED_BYTES[lay] * cells + FUSED_PML_BYTES[play] * npml
+        step_bytes = bytes_per_launch / 2
+    elif fused:
         bytes_per_launch = FUSED_BYTES[lay] * cells + FUSED_PML_BYTES[play] * npml
         step_bytes = bytes_per_launch
     else:
         bytes_per_launch = LAYOUT_BYTES[lay] * cells + PML_BYTES[play] * npml
         step_bytes = 2 * bytes_per_launch
     plain_step_bytes = PLAIN_CELL_STEP_BYTES * (cells + npml)
-    if fused:
+    if pair:
+        kname, kms = "k_pair", volt_ms
+    elif fused:
         kname, kms = ("k_step", "k_step2", "k_step4")[fused - 1], volt_ms
     else:
         kname, kms = ("k_volt", volt_ms) if volt_ms >= curr_ms else ("k_curr", curr_ms)
@@ -541,7 +549,11 @@ def main():
     if quad:
         form += ", four x cells per lane"
         zdepth = qzdepth
-    layout += f", {form} (z depth {zdepth})"
+    if pair:
+        layout += f", two timesteps per launch (k_pair, tiles of {ptile[0]} x {ptile[1]} columns, {ptile[2]} planes), " \
+                  f"single steps as {form}"
+    else:
+        layout += f", {form} (z depth {zdepth})"
     traffic = traffic_from_profile(kname, layout, n)
     plain_ceiling = HBM_PEAK_GBS * 1e9 / (plain_step_bytes / cells) / 1e6     # MCells/s
     out = {

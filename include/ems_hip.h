@@ -179,6 +179,14 @@ int ems_set_quad(ems_engine* h, int mode);
 /* on: 1 when the half steps run quads; zdepth: their z planes per workgroup */
 int ems_get_quad(const ems_engine* h, int* on, unsigned* zdepth);
 
+/* Two timesteps in one launch (k_pair), the automatic step of two-half-step
+ * engines whose only extensions are UPML and sources (step form and lane
+ * width both automatic, second copies of fields and fluxes fit): wherever no
+ * probe or dump samples the state between them; other steps run the two half
+ * steps.  Results are bit-identical.  on: 1 when active; tile: columns along
+ * x and y and planes of a workgroup; launches: pairs advanced so far. */
+int ems_get_pair(const ems_engine* h, int* on, unsigned tile[3], unsigned* launches);
+
 /* Active layouts and table sizes (known after ems_init for the UPML part):
  * layout, pml_layout: EMS_LAYOUT_PLAIN or EMS_LAYOUT_COMPRESSED (pml_layout 0
  * without UPML); n_unique / n_unique_pml: table entries (0 when plain). */
@@ -338,7 +346,8 @@ int ems_energy(ems_engine* h, double* out);
 int ems_energy_noalloc(ems_engine* h, double* d_out);
 
 /* device time of the last ems_iterate call in milliseconds (HIP events) and
- * the average duration of the voltage / current update kernels it launched */
+ * the average duration of the voltage / current update kernels it launched
+ * (of the two-timestep launches, and 0, where it ran any) */
 int ems_last_timing(ems_engine* h, double* total_ms, double* volt_ms, double* curr_ms);
 
 /* record HIP events around every voltage / current update kernel (adds one

@@ -100,6 +100,7 @@ ENGINE_API = [
     ("ems_get_field_at", C.c_int, [vp, C.c_int, C.c_int, up, C.POINTER(dp), dp]),
     ("ems_set_quad", C.c_int, [vp, C.c_int]),
     ("ems_get_quad", C.c_int, [vp, ip, up]),
+    ("ems_get_pair", C.c_int, [vp, ip, up, up]),
     ("ems_set_excitation", C.c_int, [vp, fp, fp, C.c_uint, C.c_int, C.c_uint, up, usp, fp, up,
                                      C.c_uint, up, usp, fp, up]),
     ("ems_add_upml", C.c_int, [vp, up, up, fp, fp, fp, fp, fp, fp]),

@@ -23,6 +23,7 @@
 #include <string>
 #include <unordered_map>
 #include <thread>
+#include <type_traits>
 #include <numeric>
 #include <vector>
 
@@ -2054,6 +2055,481 @@ __global__ __launch_bounds__(kBlock, 3) void k_step4t(const Step4Args ag, const 
 }
 
 // ---------------------------------------------------------------------------
+// Two timesteps in one z sweep (k_pair).  The half steps move 38 bytes a cell
+// each way through HBM and a single sweep 50 a step; here the intermediate
+// state never leaves the chip, so two steps read and write the fields once.
+//
+// A workgroup owns a tile of tx x ty columns, one per thread, and a z chunk.
+// In iteration z four updates run, each a plane behind what it needs from the
+// neighbouring columns, so that one barrier a plane serves them all:
+//   A  V^{n+1}(z)    from V^n(z), I^n(z), I^n(z-1)       (state n, from memory)
+//   B  I^{n+1}(z-1)  from I^n(z-1), V^{n+1}(z-1), V^{n+1}(z)
+//   C  V^{n+2}(z-2)  from V^{n+1}(z-2), I^{n+1}(z-2), I^{n+1}(z-3)
+//   D  I^{n+2}(z-3)  from I^{n+1}(z-3), V^{n+2}(z-3), V^{n+2}(z-2)
+// The own column's planes are carried in registers, the x and y neighbours of
+// V^{n+1}(z-1), I^{n+1}(z-2) and V^{n+2}(z-3) come from LDS, double-buffered
+// by plane (so the loop body is written twice, by parity).  B needs the next
+// column and row, C the previous one, D the next: a tile's results are valid
+// on its columns 1 .. tx-3 and rows 1 .. ty-3 (all of them at the mesh
+// edges), so tiles advance by tx-3 and ty-3 and recompute their rims; a chunk
+// starts one plane early and ends three late.  State n is read from one set
+// of buffers (fields, fluxes, timestep counter) and state n+2 written to the
+// other.  Per element the arithmetic is volt_tile / curr_tile's, sources
+// included, so results are bit-identical.
+//
+// What bounds it is the round trip of a plane, not bytes or issue: waits
+// count outstanding loads in order, so one late gather waits for everything
+// in flight.  Hence state n is loaded two planes ahead, and coefficients stay
+// in registers until a column's table entry changes.  With loads one plane
+// ahead 82 us per step at 253 x 209 x 178 and 321 us at 256^3 with UPML; as
+// it is 56 and 220 us, against 171 and 315 us in two half steps (device time
+// per step; 168 and 76 G cells/s, 4.2 and 2.3 TB/s of 50 bytes a cell and 52 a
+// UPML position per launch).  Plain stores: non-temporal ones leave the cache
+// lines shared by neighbouring tiles to be merged in memory (237 us at 256^3).
+// ---------------------------------------------------------------------------
+constexpr unsigned kPairMax = 1024;      // threads of a workgroup (columns of its tile)
+constexpr unsigned kPairMaxPml = 512;    // with UPML, whose fluxes and coefficients take 40 registers more
+constexpr unsigned kPairLds = 18;        // floats of LDS per column: 3 fields x 3 components x 2 planes
+
+// UPML of k_pair: the slab table in device memory, both sides' arrays
+struct PairPml {
+    const SlabTab* tab;
+    unsigned n;
+    unsigned long long npos;
+    const unsigned* pidx;
+    const float *coefV, *coefI;
+    const float4 *ptabV, *ptabI;
+};
+
+struct PairArgs {
+    unsigned Nx, Ny, Nz, plane;
+    unsigned long long cs;
+    unsigned tx, ty, ntx, ntiles;        // tile, tiles along x and over the plane
+    unsigned zd;                         // planes per chunk
+    CoefArgs kV, kI;
+    PairPml pml;
+    ExcArgs eV, eI;                      // lists per column, ordered by plane
+    unsigned sz[2][2];                   // first and last plane of the voltage and current sources
+    const unsigned* tmask;               // bit per tile: its columns hold a source (null: none does)
+};
+
+// buffers of one launch: state n read, state n+2 written
+struct PairBufs {
+    const float *V0, *I0, *fV0, *fI0;
+    float *V2, *I2, *fV2, *fI2;
+    const unsigned* ts_in;
+    unsigned* ts_out;
+};
+
+// the sources of plane z in the column's list [b, e), in list order
+__device__ __forceinline__ void pair_sources(const ExcArgs& ex, unsigned col, unsigned z, int ts, float f[3])
+{
+    unsigned b = ex.beg[col];
+    const unsigned e = ex.beg[col + 1];
+    for (unsigned n = e - b; n;) {                   // the first entry of plane z
+        const unsigned h = n / 2;
+        if (ex.ent[b + h].z < z) {
+            b += h + 1;
+            n -= h + 1;
+        } else n = h;
+    }
+    for (; b < e && ex.ent[b].z == z; ++b) {
+        const ExcEnt E = ex.ent[b];
+        const float sv = E.amp * ex.sig[exc_sample(ts, E.delay, ex.period, ex.length)];
+        if (E.dir == 0) f[0] = f[0] + sv;
+        else if (E.dir == 1) f[1] = f[1] + sv;
+        else f[2] = f[2] + sv;
+    }
+}
+
+__device__ __forceinline__ float ldb(const float* __restrict__ b, unsigned off)
+{
+    return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(b) + off);
+}
+
+__device__ __forceinline__ void stb(float* b, unsigned off, float v)
+{
+    *reinterpret_cast<float*>(reinterpret_cast<char*>(b) + off) = v;
+}
+
+// coefficients of the cell at byte offset off (table entry u)
+template <bool CC>
+__device__ __forceinline__ void pair_coef(const CoefArgs& k, unsigned long long cs, unsigned off, unsigned u, float a[3],
+                                          float b[3])
+{
+    if (CC) {
+        const char* t = reinterpret_cast<const char*>(k.tab) + (u << 5);
+        const float4 t0 = *reinterpret_cast<const float4*>(t);
+        const float2 t1 = *reinterpret_cast<const float2*>(t + 16);
+        a[0] = t0.x; b[0] = t0.y;
+        a[1] = t0.z; b[1] = t0.w;
+        a[2] = t1.x; b[2] = t1.y;
+    } else {
+#pragma unroll
+        for (int n = 0; n < 3; ++n) {
+            a[n] = ldb(k.cc + n * cs, off);
+            b[n] = ldb(k.cv + n * cs, off);
+        }
+    }
+}
+
+// A copy that the compiler keeps as one.  Merged with its source, a register
+// about to be loaded again, it would instead copy (and so wait for) the
+// load's result at the end of the loop; and values gathered in a branch are
+// waited for there and not after it, where the wait would cover every load
+// in flight on the path without the gather too.
+template <class V>
+__device__ __forceinline__ V keep(V v)
+{
+    V r;
+    asm("v_mov_b32 %0, %1" : "=v"(r) : "v"(v));
+    return r;
+}
+
+// UPML coefficients of one cell and side
+struct PairPmlK {
+    float k0[3], ko[3], kn[3];
+    unsigned at = ~0u;             // table entry (compressed) or position (plain) they belong to
+};
+
+template <int PM>
+__device__ __forceinline__ void pair_pml_load(unsigned li, unsigned px, unsigned long long npos, const float* coef,
+                                              const float4* ptab, float k[9])
+{
+    if (PM == kPmlPlain) {
+#pragma unroll
+        for (int n = 0; n < 9; ++n) k[n] = ldb(coef + n * npos, 4u * li);
+    } else {
+        const char* t = reinterpret_cast<const char*>(ptab) + 48u * px;
+        const float4 t0 = *reinterpret_cast<const float4*>(t), t1 = *reinterpret_cast<const float4*>(t + 16);
+        k[0] = t0.x; k[1] = t0.y; k[2] = t0.z;
+        k[3] = t0.w; k[4] = t1.x; k[5] = t1.y;
+        k[6] = t1.z; k[7] = t1.w; k[8] = *reinterpret_cast<const float*>(t + 32);
+    }
+}
+
+// one cell's update: x0 its old values, fl its UPML flux (updated), pml: it
+// has one.  main: the main update covers it.
+template <int PM>
+__device__ __forceinline__ void pair_cell(const float x0[3], const float a[3], const float b[3], const float curl[3],
+                                          bool pml, const PairPmlK& K, float fl[3], bool main, float out[3])
+{
+    float f[3];
+#pragma unroll
+    for (int n = 0; n < 3; ++n) {
+        const float xin = PM != kNoPml && pml ? fl[n] : x0[n];
+        f[n] = xin * a[n];
+        f[n] = f[n] + b[n] * curl[n];
+        if (!main) f[n] = xin;
+    }
+    if (PM != kNoPml && pml) {
+#pragma unroll
+        for (int n = 0; n < 3; ++n) {
+            const float t = K.k0[n] * x0[n] - K.ko[n] * fl[n];
+            fl[n] = f[n];
+            f[n] = t + K.kn[n] * f[n];
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < 3; ++n) out[n] = f[n];
+}
+
+// the workgroup's sweep; SRC: its columns hold sources
+template <int PM, bool CC, bool LT, bool SRC>
+__device__ __forceinline__ void pair_sweep(const PairArgs& ag, const PairBufs& B, const CoefArgs& kV, const CoefArgs& kI,
+                                           float* s, unsigned tile, unsigned zc, int ts)
+{
+    const unsigned T = blockDim.x, tid = threadIdx.x;
+    const unsigned long long cs = ag.cs, npos = ag.pml.npos;
+    const unsigned X0 = tile % ag.ntx * (ag.tx - 3u), Y0 = tile / ag.ntx * (ag.ty - 3u);
+    const unsigned ly = tid / ag.tx, lx = tid - ly * ag.tx;
+    const bool in = ly < ag.ty && X0 + lx < ag.Nx && Y0 + ly < ag.Ny;
+    // threads past the tile or the mesh work on a clamped column and store nothing
+    const unsigned x = min(X0 + lx, ag.Nx - 1u), y = min(Y0 + ly, ag.Ny - 1u);
+    const bool own = in && (lx || !x) && (ly || !y) && (lx + 2u < ag.tx || X0 + ag.tx >= ag.Nx) &&
+                     (ly + 2u < ag.ty || Y0 + ag.ty >= ag.Ny);
+    const unsigned col = x + ag.Nx * y;
+    const bool cmain = x + 1u < ag.Nx && y + 1u < ag.Ny;
+    const unsigned z0 = zc * ag.zd, z1 = min(z0 + ag.zd, ag.Nz), zl = ag.Nz - 1u;
+    const unsigned zs = z0 ? z0 - 1u : 0u;                       // first plane of A and B
+    const unsigned zA = min(z1 + 1u, zl);                        // last plane of A
+    // byte offsets: the column, its x-1 and y-1 neighbours (itself at 0)
+    const unsigned P4 = 4u * ag.plane, c4 = 4u * col;
+    const unsigned xm = x ? 4u : 0u, ym = y ? 4u * ag.Nx : 0u;
+    // the neighbours' LDS slots (the own one where there is no valid neighbour)
+    const unsigned nxm = lx ? tid - 1u : tid, nxp = tid + 1u < T ? tid + 1u : tid;
+    const unsigned nym = ly ? tid - ag.tx : tid, nyp = tid + ag.tx < T ? tid + ag.tx : tid;
+    const float *Vx = B.V0, *Vy = B.V0 + cs, *Vz = B.V0 + 2 * cs, *Ix = B.I0, *Iy = B.I0 + cs, *Iz = B.I0 + 2 * cs;
+    // the column's UPML positions up to plane pend: pbase + z * pstep, or none
+    unsigned pend = 0, pbase = 0, pstep = 0;
+    bool pon = false;
+    // state n of the next two planes, by iteration parity: loaded two
+    // iterations ahead, for the latency of HBM
+    float pv[2][3], pi[2][3], pn[2][4], pf[2][3], qf[2][3];
+    unsigned pu[2] = {0, 0}, pl[2] = {~0u, ~0u}, px[2] = {0, 0};
+    auto fetch = [&](auto par, unsigned z) {
+        constexpr int P = decltype(par)::value;
+        const unsigned o = c4 + z * P4;
+        if (CC) pu[P] = ag.kV.idx[o >> 2];
+        pi[P][0] = ldb(Ix, o);
+        pi[P][1] = ldb(Iy, o);
+        pi[P][2] = ldb(Iz, o);
+        pn[P][0] = ldb(Iz, o - ym);
+        pn[P][1] = ldb(Ix, o - ym);
+        pn[P][2] = ldb(Iz, o - xm);
+        pn[P][3] = ldb(Iy, o - xm);
+        pv[P][0] = ldb(Vx, o);
+        pv[P][1] = ldb(Vy, o);
+        pv[P][2] = ldb(Vz, o);
+        if (PM != kNoPml) {
+            if (z >= pend) {
+                // the slab that holds plane z of the column, and the plane where that changes
+                pend = ag.Nz;
+                pon = false;
+                for (unsigned k = 0; k < ag.pml.n; ++k) {
+                    const SlabTab S = ag.pml.tab[k];
+                    if ((int)x < S.x0 || (int)x > S.x1 || (int)y < S.y0 || (int)y > S.y1) continue;
+                    if ((int)z < S.z0) pend = min(pend, (unsigned)S.z0);
+                    else if ((int)z <= S.z1) {
+                        pend = (unsigned)S.z1 + 1u;
+                        pstep = S.nx * S.ny;
+                        pbase = (unsigned)S.off + (x - (unsigned)S.xo) + S.nx * (y - (unsigned)S.y0) - pstep * (unsigned)S.z0;
+                        pon = true;
+                        break;
+                    }
+                }
+            }
+            pl[P] = ~0u;
+            if (pon) {
+                pl[P] = pbase + z * pstep;
+                if (PM == kPmlCompressed) px[P] = ag.pml.pidx[pl[P]];
+#pragma unroll
+                for (int n = 0; n < 3; ++n) pf[P][n] = ldb(B.fV0 + n * npos, 4u * pl[P]);
+            }
+        }
+    };
+    // B's flux of the plane whose position is l
+    auto fetch_i = [&](auto par, unsigned l) {
+        constexpr int P = decltype(par)::value;
+        if (PM != kNoPml && l != ~0u) {
+#pragma unroll
+            for (int n = 0; n < 3; ++n) qf[P][n] = ldb(B.fI0 + n * npos, 4u * l);
+        }
+    };
+    // carried values, by iteration parity: at iteration z slot P holds
+    // V^{n+1}(z-2), I^{n+1}(z-3) and the UPML fluxes of those, slot 1-P
+    // V^{n+1}(z-1), I^{n+1}(z-2), V^{n+2}(z-3)
+    float v1[2][3] = {}, i1[2][3] = {}, v2[2][3] = {}, i0[3] = {}, fv[2][3], fi[2][3];
+    unsigned u1 = 0, u2 = 0, u3 = 0, l1 = ~0u, l2 = ~0u, l3 = ~0u, x1 = 0;
+    // coefficients: A's and B's, by parity, serve C and D two iterations later.
+    // A column's table entries are gathered only where they change (a material
+    // boundary, the graded planes): a gather waits for every load in flight.
+    // From an LDS table one set serves all four updates.
+    constexpr int S = LT ? 1 : 2;
+    float aV[S][3], bV[S][3], aI[S][3], bI[S][3];
+    unsigned hV[S], hI[S];
+#pragma unroll
+    for (int k = 0; k < S; ++k) hV[k] = hI[k] = ~0u;
+    PairPmlK kpV[2], kpI[2];
+    auto lds_coef = [&](const CoefArgs& k, unsigned u, unsigned& h, float a[3], float b[3]) {
+        if (u == h) return;
+        h = u;
+        pair_coef<true>(k, cs, 0u, u, a, b);
+    };
+    if (zs) {
+        i0[0] = ldb(Ix, c4 + (zs - 1u) * P4);
+        i0[1] = ldb(Iy, c4 + (zs - 1u) * P4);
+    }
+    const std::integral_constant<int, 0> even{};
+    const std::integral_constant<int, 1> odd{};
+    // (in this order, as in the loop: waits count the loads issued since)
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(even, zs);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(odd, min(zs + 1u, zA));
+    fetch_i(odd, pl[0]);
+    __builtin_amdgcn_sched_barrier(0);
+    // Every iteration runs all four updates: before a plane's first and after
+    // its last valid one they work on clamped planes, and nothing reads or
+    // stores the result.
+    auto iter = [&](auto par, const unsigned z) {
+        constexpr int P = decltype(par)::value, Q = 1 - P;
+        float* w = s + P * 9u * T + tid;                         // written this iteration
+        const float* r = s + Q * 9u * T;                         // written in the previous one
+        const unsigned zb = z - 1u, zv = z - 2u, zi = z - 3u;
+        const unsigned oa = c4 + min(z, zl) * P4, ob = c4 + min(z ? zb : 0u, zl) * P4;
+        const unsigned oc = c4 + min(z > 1u ? zv : 0u, zl) * P4, od = c4 + min(z > 2u ? zi : 0u, zl) * P4;
+        float curl[3], i2[3];
+        // ---- C: V^{n+2}(z-2)
+        {
+            if (LT) lds_coef(kV, u2, hV[0], aV[0], bV[0]);
+            const float iz_ym = r[5 * T + nym], ix_ym = r[3 * T + nym], iz_xm = r[5 * T + nxm], iy_xm = r[4 * T + nxm];
+            const float iy_zm = zv ? i1[P][1] : i1[Q][1], ix_zm = zv ? i1[P][0] : i1[Q][0];
+            curl[0] = i1[Q][2] - iz_ym - i1[Q][1] + iy_zm;
+            curl[1] = i1[Q][0] - ix_zm - i1[Q][2] + iz_xm;
+            curl[2] = i1[Q][1] - iy_xm - i1[Q][0] + ix_ym;
+            pair_cell<PM>(v1[P], aV[LT ? 0 : P], bV[LT ? 0 : P], curl, l2 != ~0u, kpV[P], fv[P], true, v2[P]);
+            if (SRC && zv >= ag.sz[0][0] && zv <= ag.sz[0][1]) pair_sources(ag.eV, col, zv, ts + 1, v2[P]);
+        }
+        // ---- D: I^{n+2}(z-3)
+        {
+            if (LT) lds_coef(kI, u3, hI[0], aI[0], bI[0]);
+            const float vz_yp = r[8 * T + nyp], vx_yp = r[6 * T + nyp], vz_xp = r[8 * T + nxp], vy_xp = r[7 * T + nxp];
+            curl[0] = v2[Q][2] - vz_yp - v2[Q][1] + v2[P][1];
+            curl[1] = v2[Q][0] - v2[P][0] - v2[Q][2] + vz_xp;
+            curl[2] = v2[Q][1] - vy_xp - v2[Q][0] + vx_yp;
+            pair_cell<PM>(i1[P], aI[LT ? 0 : P], bI[LT ? 0 : P], curl, l3 != ~0u, kpI[P], fi[P], cmain && zi < zl, i2);
+            if (SRC && zi >= ag.sz[1][0] && zi <= ag.sz[1][1]) pair_sources(ag.eI, col, zi, ts + 1, i2);
+        }
+        if (own && zv >= z0 && zv < z1) {
+#pragma unroll
+            for (int n = 0; n < 3; ++n) stb(B.V2 + n * cs, oc, v2[P][n]);
+            if (PM != kNoPml && l2 != ~0u) {
+#pragma unroll
+                for (int n = 0; n < 3; ++n) stb(B.fV2 + n * npos, 4u * l2, fv[P][n]);
+            }
+        }
+        if (own && z >= z0 + 3u && zi < z1) {
+#pragma unroll
+            for (int n = 0; n < 3; ++n) stb(B.I2 + n * cs, od, i2[n]);
+            if (PM != kNoPml && l3 != ~0u) {
+#pragma unroll
+                for (int n = 0; n < 3; ++n) stb(B.fI2 + n * npos, 4u * l3, fi[P][n]);
+            }
+        }
+        // coefficients of A and B, in one round trip
+        if (!LT || PM != kNoPml) {
+            const bool pA = PM != kNoPml && pl[P] != ~0u, pB = PM != kNoPml && l1 != ~0u;
+            const unsigned tA = PM == kPmlPlain ? pl[P] : px[P], tB = PM == kPmlPlain ? l1 : x1;
+            const bool gm = !LT && (!CC || pu[P] != hV[LT ? 0 : P] || u1 != hI[LT ? 0 : P]);
+            const bool gp = PM != kNoPml && ((pA && tA != kpV[P].at) || (pB && tB != kpI[P].at));
+            if (gm || gp) {
+                float ca[3], cb[3], da[3], db[3], k[9], q[9];
+                if (!LT) {
+                    pair_coef<CC>(kV, cs, oa, pu[P], ca, cb);
+                    pair_coef<CC>(kI, cs, ob, u1, da, db);
+                }
+                if (pA) pair_pml_load<PM>(pl[P], px[P], npos, ag.pml.coefV, ag.pml.ptabV, k);
+                if (pB) pair_pml_load<PM>(l1, x1, npos, ag.pml.coefI, ag.pml.ptabI, q);
+                if (!LT) {
+                    hV[LT ? 0 : P] = pu[P];
+                    hI[LT ? 0 : P] = u1;
+#pragma unroll
+                    for (int n = 0; n < 3; ++n) {
+                        aV[LT ? 0 : P][n] = keep(ca[n]);
+                        bV[LT ? 0 : P][n] = keep(cb[n]);
+                        aI[LT ? 0 : P][n] = keep(da[n]);
+                        bI[LT ? 0 : P][n] = keep(db[n]);
+                    }
+                }
+                if (pA) {
+                    kpV[P].at = tA;
+#pragma unroll
+                    for (int n = 0; n < 3; ++n) {
+                        kpV[P].k0[n] = keep(k[n]);
+                        kpV[P].ko[n] = keep(k[3 + n]);
+                        kpV[P].kn[n] = keep(k[6 + n]);
+                    }
+                }
+                if (pB) {
+                    kpI[P].at = tB;
+#pragma unroll
+                    for (int n = 0; n < 3; ++n) {
+                        kpI[P].k0[n] = keep(q[n]);
+                        kpI[P].ko[n] = keep(q[3 + n]);
+                        kpI[P].kn[n] = keep(q[6 + n]);
+                    }
+                }
+            }
+        }
+        // ---- A: V^{n+1}(z)
+        {
+            if (LT) lds_coef(kV, pu[P], hV[0], aV[0], bV[0]);
+            const float iy_zm = z ? i0[1] : pi[P][1], ix_zm = z ? i0[0] : pi[P][0];
+            curl[0] = pi[P][2] - pn[P][0] - pi[P][1] + iy_zm;
+            curl[1] = pi[P][0] - ix_zm - pi[P][2] + pn[P][2];
+            curl[2] = pi[P][1] - pn[P][3] - pi[P][0] + pn[P][1];
+            pair_cell<PM>(pv[P], aV[LT ? 0 : P], bV[LT ? 0 : P], curl, pl[P] != ~0u, kpV[P], pf[P], true, v1[P]);
+            if (SRC && z >= ag.sz[0][0] && z <= ag.sz[0][1]) pair_sources(ag.eV, col, z, ts, v1[P]);
+        }
+        // ---- B: I^{n+1}(z-1)
+        {
+            if (LT) lds_coef(kI, u1, hI[0], aI[0], bI[0]);
+            const float vz_yp = r[2 * T + nyp], vx_yp = r[nyp], vz_xp = r[2 * T + nxp], vy_xp = r[T + nxp];
+            curl[0] = v1[Q][2] - vz_yp - v1[Q][1] + v1[P][1];
+            curl[1] = v1[Q][0] - v1[P][0] - v1[Q][2] + vz_xp;
+            curl[2] = v1[Q][1] - vy_xp - v1[Q][0] + vx_yp;
+            pair_cell<PM>(i0, aI[LT ? 0 : P], bI[LT ? 0 : P], curl, l1 != ~0u, kpI[P], qf[P], cmain && zb < zl, i1[P]);
+            if (SRC && zb >= ag.sz[1][0] && zb <= ag.sz[1][1]) pair_sources(ag.eI, col, zb, ts, i1[P]);
+        }
+#pragma unroll
+        for (int n = 0; n < 3; ++n) {
+            w[n * T] = v1[P][n];
+            w[(3 + n) * T] = i1[P][n];
+            w[(6 + n) * T] = v2[P][n];
+            i0[n] = keep(pi[P][n]);
+            if (PM != kNoPml) {
+                fv[P][n] = keep(pf[P][n]);
+                fi[P][n] = keep(qf[P][n]);
+            }
+        }
+        if (LT) {
+            u3 = u2;
+            u2 = u1;
+        }
+        u1 = keep(pu[P]);
+        if (PM != kNoPml) {
+            l3 = l2; l2 = l1; l1 = keep(pl[P]);
+            x1 = keep(px[P]);
+        }
+        fetch(par, min(z + 2u, zA));
+        fetch_i(par, pl[Q]);
+        __syncthreads();
+    };
+    // planes zs .. z1+2 (and one past where their number is odd: a mid-loop
+    // exit made the compiler copy, and so wait for, the loads just issued)
+    for (unsigned z = zs; z <= z1 + 2u; z += 2u) {
+        iter(even, z);
+        iter(odd, z + 1u);
+    }
+}
+
+template <int PM, bool CC, bool LT>
+__global__ __launch_bounds__(PM == kNoPml ? kPairMax : kPairMaxPml) void k_pair(const PairArgs ag, const PairBufs B)
+{
+    extern __shared__ float4 s_tab[];
+    CoefArgs kV = ag.kV, kI = ag.kI;
+    float* s = reinterpret_cast<float*>(s_tab);
+    if (LT) {
+        stage_table(s_tab, ag.kV.tab, ag.kV.ntab);
+        stage_table(s_tab + ag.kV.ntab, ag.kI.tab, ag.kI.ntab);
+        kV.tab = s_tab;
+        kI.tab = s_tab + ag.kV.ntab;
+        s = reinterpret_cast<float*>(s_tab + ag.kV.ntab + ag.kI.ntab);
+        __syncthreads();
+    }
+    const int ts = (int)B.ts_in[0];
+    if (blockIdx.x == 0 && threadIdx.x == 0) B.ts_out[0] = (unsigned)ts + 2u;
+    const unsigned bid = xcd_tile(blockIdx.x, gridDim.x);
+    const unsigned tile = bid % ag.ntiles, zc = bid / ag.ntiles;
+    // the leanest sweep for what the workgroup's cells hold
+    const bool src = ag.tmask && (ag.tmask[tile >> 5] >> (tile & 31u) & 1u);
+    bool pml = false;
+    if (PM != kNoPml) {
+        const int X0 = (int)(tile % ag.ntx * (ag.tx - 3u)), Y0 = (int)(tile / ag.ntx * (ag.ty - 3u));
+        const int za = (int)(zc * ag.zd) - 1, zb = (int)((zc + 1u) * ag.zd) + 1;
+        for (unsigned k = 0; k < ag.pml.n; ++k) {
+            const SlabTab& S = ag.pml.tab[k];
+            pml = pml || (X0 <= S.x1 && X0 + (int)ag.tx > S.x0 && Y0 <= S.y1 && Y0 + (int)ag.ty > S.y0 && za <= S.z1 &&
+                          zb >= S.z0);
+        }
+    }
+    if (src) pair_sweep<PM, CC, LT, true>(ag, B, kV, kI, s, tile, zc, ts);
+    else if (PM != kNoPml && pml) pair_sweep<PM, CC, LT, false>(ag, B, kV, kI, s, tile, zc, ts);
+    else pair_sweep<kNoPml, CC, LT, false>(ag, B, kV, kI, s, tile, zc, ts);
+}
+
+// ---------------------------------------------------------------------------
 // ++numTS after a single-sweep step (Engine::IterateTS, FDTD/engine.cpp:283).
 // Every workgroup of the step reads the counter, so the step itself cannot
 // advance it; a one-thread launch after it does, with no fence or atomic
@@ -3152,6 +3628,15 @@ struct ems_engine {
     unsigned* mur_rim[2] = {nullptr, nullptr};    // their rim points (y or z within 2 lines of the mesh edge)
     unsigned nrim[2] = {0, 0};
     ExcArgs eV{}, eI{};
+    // two timesteps per launch (k_pair) where no sample falls between them;
+    // the arguments that stay the same, the second timestep counter
+    bool pair = false;
+    PairArgs pargs{};
+    unsigned pair_threads = 0, pair_blocks = 0;
+    size_t pair_lds = 0;
+    bool pair_lt = false;
+    unsigned* numts_alt = nullptr;
+    unsigned pair_launches = 0;
     int pml_mode = kNoPml;
     unsigned n_unique_pml = 0;
     // Mur faces in creation order
@@ -3222,6 +3707,7 @@ struct ems_engine {
         hipGraph_t graph = nullptr;
         hipGraphExec_t exec = nullptr;
         size_t nalloc = 0;                // device allocations of the engine when captured
+        unsigned pairs = 0;               // launches of k_pair in it
     };
     unsigned graph_chunk = 32;            // requested steps per graph (0: direct launches)
     unsigned graph_len = 0;               // steps per graph of the captured set
@@ -4381,6 +4867,211 @@ static int setup_vsrc(ems_engine* h)
 
 }  // extern "C"
 
+// Tile and chunk of k_pair.  A CU holds `waves` wavefronts of the kernel and
+// its LDS.  A plane of a workgroup takes at least its round trip (LDS
+// exchange, barrier, the loads that did not arrive) and, with the CU full,
+// its share of issue and memory time, which grows as rows get short: every
+// row of a tile starts and ends inside a cache line.  Measured per plane and
+// 1024 columns: 2.81, 2.09, 1.76 us at 39, 64 and 128 columns a row (253 x
+// 209 x 178 cavity, from HBM), and with UPML 2.49, 2.38, 2.05, 1.65 us per
+// 512 at 23, 36, 53 and 102.  The estimate adds the planes and columns that
+// neighbours compute twice and the last, partly empty round of workgroups;
+// the smallest wins.
+// tiles of t lines, advancing by t-3, that cover n lines
+static unsigned pair_tiles(unsigned n, unsigned t) { return n <= t ? 1u : (n - 3u + t - 4u) / (t - 3u); }
+
+struct PairCost {
+    double lat, issue, row;        // us: a plane's round trip; per 1024 columns; and that over the row length
+};
+constexpr PairCost kPairPlain{0.9, 1.3, 59.0}, kPairUpml{1.5, 2.8, 50.0};
+static void choose_pair_tile(const unsigned N[3], const PairCost& cost, unsigned most, unsigned column, unsigned waves,
+                             size_t table, unsigned cus, PairArgs& a)
+{
+    double best = 1e300;
+    // lines per tile that cover n lines evenly with k tiles
+    auto even = [](unsigned n, unsigned k) { return k == 1 ? n : (n - 3u + k - 1u) / k + 3u; };
+    unsigned ltx = 0;
+    for (unsigned kx = 1; kx <= N[0]; ++kx) {
+        const unsigned tx = even(N[0], kx), nx = pair_tiles(N[0], tx);
+        if (tx < std::min(N[0], 24u)) break;
+        if (tx == ltx || tx > 256) continue;
+        ltx = tx;
+        unsigned lty = 0;
+        for (unsigned ky = 1; ky <= N[1]; ++ky) {
+            const unsigned ty = even(N[1], ky), ny = pair_tiles(N[1], ty);
+            if (ty < std::min(N[1], 6u)) break;
+            if (ty == lty) continue;
+            lty = ty;
+            const unsigned T = (tx * ty + 63u) / 64u * 64u;
+            const size_t lds = (size_t)column * T + table;
+            if (T > most || lds > 160u * 1024u) continue;
+            const unsigned res = std::min(waves / (T / 64u), (unsigned)(160u * 1024u / lds));
+            if (!res) continue;
+            unsigned last = 0;
+            for (unsigned nz = 1; nz <= N[2]; ++nz) {
+                const unsigned zd = (N[2] + nz - 1) / nz;
+                if (zd == last) continue;
+                last = zd;
+                if (zd < 2 && N[2] > 2) break;
+                const unsigned long long wg = (unsigned long long)nx * ny * ((N[2] + zd - 1) / zd);
+                const unsigned long long rounds = (wg + (unsigned long long)cus * res - 1) / ((unsigned long long)cus * res);
+                const double full = (double)std::min<unsigned long long>(res, (wg + cus - 1) / cus) * T / kPairMax;
+                const double c = (double)rounds * (zd + 5) * std::max(cost.lat, (cost.issue + cost.row / tx) * full);
+                if (c < best) {
+                    best = c;
+                    a.tx = tx;
+                    a.ty = ty;
+                    a.ntx = nx;
+                    a.ntiles = nx * ny;
+                    a.zd = zd;
+                }
+            }
+        }
+    }
+}
+
+template <int PM>
+static const void* pair_kernel(bool cmp, bool lt)
+{
+    if (!cmp) return (const void*)k_pair<PM, false, false>;
+    return lt ? (const void*)k_pair<PM, true, true> : (const void*)k_pair<PM, true, false>;
+}
+
+static const void* pair_kernel(const ems_engine* h, bool lt)
+{
+    const int pm = h->pmlV.n ? h->pml_mode : kNoPml;
+    return pm == kPmlCompressed ? pair_kernel<kPmlCompressed>(h->cmp, lt)
+           : pm == kPmlPlain    ? pair_kernel<kPmlPlain>(h->cmp, lt)
+                                : pair_kernel<kNoPml>(h->cmp, lt);
+}
+
+// Two timesteps per launch (k_pair): the automatic step of meshes whose only
+// extensions are UPML and sources (Mur, Lorentz, lumped RLC and steady-state
+// detection have hooks between the half steps), where neither the step form
+// nor the lane width was asked for, 32-bit byte offsets reach every cell and
+// the second copy of fields and fluxes fits with 1 GiB to spare.  With UPML
+// from a million cells on: per step 32.3 -> 24.8 us at 109 x 97 x 131, 60 ->
+// 49 us at 160 x 150 x 140, 315 -> 220 us at 256^3, but 20.9 -> 21.9 us at
+// 90^3 and 10.5 -> 13.4 us at 64^3, where a workgroup sweeps few planes and
+// most of them are graded.  Without UPML at every size: 7.2 -> 5.6 us at
+// 64^3, 34.5 -> 17.3 us at 140^3, 96 -> 57 us at 253 x 209 x 178 (plain
+// accesses; 170 us as it ran).
+constexpr unsigned long long kPairUpmlCells = 1000000;
+static int setup_pair(ems_engine* h)
+{
+    h->pair = false;
+    const unsigned* N = h->N;
+    bool on = (!h->fused || h->fused == 3) && h->fused_req == -1 && h->quad_req == -1 && h->mur.empty() &&
+              h->lor.empty() && h->rlc.empty() && !h->has_ss && N[0] < 65535 && N[1] < 65535 && N[2] < 65535 &&
+              N[0] >= 4 && N[1] >= 4 && N[2] >= 2 && h->cs < (1ull << 30) && h->pmlV.npos < (1ull << 30);
+    bool big = !h->pmlV.n || (unsigned long long)h->g.plane * N[2] >= kPairUpmlCells;
+    for (int c = 0; c < 2; ++c) on = on && h->exc[c].host.size() == h->exc[c].K;
+    if (const char* e = std::getenv("EMS_PAIR")) big = std::atoi(e) != 0;
+    if (!on || !big) return 0;
+    const size_t np = h->pmlV.n ? h->pmlV.npos : 0;
+    size_t freeb = 0, totalb = 0;
+    const size_t need = 6 * ((h->fused ? 0 : h->cs) + np) * sizeof(float) + (1ull << 30);
+    if (hipMemGetInfo(&freeb, &totalb) != hipSuccess || freeb < need) return 0;
+    PairArgs& a = h->pargs;
+    a = PairArgs{};
+    a.Nx = N[0];
+    a.Ny = N[1];
+    a.Nz = N[2];
+    a.plane = h->g.plane;
+    a.cs = h->cs;
+    a.kV = h->kV;
+    a.kI = h->kI;
+    int rc;
+    if (np) {
+        SlabTab* tab;
+        if ((rc = upload(h, &tab, h->pmlV.tab, (size_t)h->pmlV.n))) return rc;
+        a.pml = PairPml{tab, (unsigned)h->pmlV.n, h->pmlV.npos, h->pmlV.pidx, h->pmlV.coef, h->pmlI.coef, h->pmlV.ptab, h->pmlI.ptab};
+    }
+    // both sides' tables in LDS where they leave it room for the tiles
+    size_t table = h->cmp ? (size_t)(h->kV.ntab + h->kI.ntab) * sizeof(float4) : 0;
+    const bool lt = h->cmp && table <= kLdsTabBytes;
+    if (!lt) table = 0;
+    const void* k = pair_kernel(h, lt);
+    const unsigned most = np ? kPairMaxPml : kPairMax;
+    const unsigned lds = kPairLds * (unsigned)sizeof(float);       // per column
+    hipFuncAttributes fa{};
+    HIPCHK(hipFuncGetAttributes(&fa, k));
+    const unsigned waves = std::min(32u, 4u * (512u / std::max(8u, ((unsigned)fa.numRegs + 7u) / 8u * 8u)));
+    hipDeviceProp_t prop;
+    HIPCHK(hipGetDeviceProperties(&prop, h->device));
+    choose_pair_tile(N, np ? kPairUpml : kPairPlain, most, lds, waves, table, (unsigned)prop.multiProcessorCount, a);
+    if (const char* e = std::getenv("EMS_PAIR_TILE")) {
+        unsigned tx, ty, zd;
+        if (std::sscanf(e, "%u,%u,%u", &tx, &ty, &zd) == 3 && tx >= 4 && ty >= 4 && tx * ty <= most && zd >= 1) {
+            a.tx = std::min(tx, N[0]);
+            a.ty = std::min(ty, N[1]);
+            a.zd = std::min(zd, N[2]);
+            a.ntx = pair_tiles(N[0], a.tx);
+            a.ntiles = a.ntx * pair_tiles(N[1], a.ty);
+        }
+    }
+    if (!a.tx) return 0;
+    h->pair_threads = (a.tx * a.ty + 63u) / 64u * 64u;
+    h->pair_blocks = a.ntiles * ((N[2] + a.zd - 1) / a.zd);
+    h->pair_lds = (size_t)lds * h->pair_threads + table;
+    HIPCHK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->pair_lds));
+    // sources: lists per column ordered by plane, their planes, and the tiles
+    // (rims included) that hold one
+    std::vector<unsigned> mask((a.ntiles + 31) / 32, 0u);
+    bool any = false;
+    for (int c = 0; c < 2; ++c) {
+        const auto& host = h->exc[c].host;
+        a.sz[c][0] = 1;
+        a.sz[c][1] = 0;
+        if (host.empty()) continue;
+        any = true;
+        std::vector<ExcEnt> ent(host);
+        std::stable_sort(ent.begin(), ent.end(), [&](const ExcEnt& l, const ExcEnt& r) {
+            const unsigned cl = l.x + N[0] * (unsigned)l.y, cr = r.x + N[0] * (unsigned)r.y;
+            return cl != cr ? cl < cr : l.z < r.z;
+        });
+        std::vector<unsigned> beg(h->g.plane + 1, 0);
+        unsigned lo = ~0u, hi = 0;
+        for (const auto& e : ent) {
+            ++beg[e.x + N[0] * (unsigned)e.y + 1];
+            lo = std::min(lo, (unsigned)e.z);
+            hi = std::max(hi, (unsigned)e.z);
+            for (unsigned t = 0; t < a.ntiles; ++t) {
+                const unsigned X0 = t % a.ntx * (a.tx - 3u), Y0 = t / a.ntx * (a.ty - 3u);
+                if (e.x >= X0 && e.x < X0 + a.tx && e.y >= Y0 && e.y < Y0 + a.ty) mask[t >> 5] |= 1u << (t & 31);
+            }
+        }
+        for (size_t i = 1; i < beg.size(); ++i) beg[i] += beg[i - 1];
+        a.sz[c][0] = lo;
+        a.sz[c][1] = hi;
+        unsigned* db;
+        ExcEnt* de;
+        if ((rc = upload(h, &db, beg.data(), beg.size())) || (rc = upload(h, &de, ent.data(), ent.size()))) return rc;
+        (c ? a.eI : a.eV) = ExcArgs{db, de, h->sig[c], h->sigLen, h->period, nullptr};
+    }
+    if (any) {
+        unsigned* dm;
+        if ((rc = upload(h, &dm, mask.data(), mask.size()))) return rc;
+        a.tmask = dm;
+    }
+    // every pair writes all of state n+2 (UPML padding positions stay zero);
+    // the quad sweep has its second buffers already
+    if (!h->fused) {
+        if ((rc = h->alloc(&h->V_alt, 3 * h->cs)) || (rc = h->alloc(&h->I_alt, 3 * h->cs))) return rc;
+        HIPCHK(hipMemset(h->V_alt, 0, 3 * h->cs * sizeof(float)));
+        HIPCHK(hipMemset(h->I_alt, 0, 3 * h->cs * sizeof(float)));
+    }
+    for (int side = 0; side < 2 && np; ++side) {
+        if ((rc = h->alloc(&h->flux_alt[side], 3 * np))) return rc;
+        HIPCHK(hipMemset(h->flux_alt[side], 0, 3 * np * sizeof(float)));
+    }
+    HIPCHK(hipDeviceSynchronize());
+    h->numts_alt = h->numts_dev + 2;
+    h->V_base = h->V;
+    h->pair = true;
+    return 0;
+}
+
 // ---------------------------------------------------------------------------
 // Hook launches (k_hooks): the jobs of a phase in the reference's order, each
 // put into the phase's last launch unless it touches a field element that a
@@ -4459,50 +5150,54 @@ static int build_hook_launches(ems_engine* h, const std::vector<HookPlan>& jobs,
         closed = (int)j == alone;
         if (closed && at) *at = (int)sets.size() - 1;
     }
+    std::vector<HookJob> d;
     for (const auto& set : sets) {
         HookLaunch L{};
-        std::vector<HookJob> d;
         for (const HookPlan* q : set) {
             L.first[L.n++] = L.nblk;
             L.nblk += (q->d.n + kBlock - 1) / kBlock;
             d.push_back(q->d);
         }
-        HookJob* dj;
-        int rc = upload(h, &dj, d.data(), d.size());
-        if (rc) return rc;
-        L.jobs = dj;
         out.push_back(L);
     }
-    return 0;
+    if (d.empty()) return 0;
+    HookJob* dj;
+    int rc = upload(h, &dj, d.data(), d.size());
+    for (auto& L : out) {
+        L.jobs = dj;
+        dj += L.n;
+    }
+    return rc;
 }
 
 // earlier faces (bit: creation index) that set the P (c = 0) or PP component
-// of each of face k's points too; null where there is none
-static int mur_over(ems_engine* h, int k, int c, const unsigned char** out)
+// of each of face k's points too, appended to `all`; its offset there, or -1
+// where there is none
+static long mur_over(const ems_engine* h, int k, int c, std::vector<unsigned char>& all)
 {
-    *out = nullptr;
-    if (h->mur.size() > kMurMaskFaces) return 0;
+    if (h->mur.size() > kMurMaskFaces) return -1;
     const auto& G = h->mur_geo[k];
     const int nP = (G.ny + 1) % 3, nPP = (G.ny + 2) % 3, comp = c ? nPP : nP;
     const MurDev& m = h->mur[k];
     const bool tr = nP < nPP;             // device order of the points (ems_add_mur)
-    std::vector<unsigned char> over((size_t)m.na * m.nb, 0);
-    bool any = false;
+    const size_t at = all.size();
     for (int j = 0; j < k; ++j) {
         const auto& J = h->mur_geo[j];
         if (J.ny == comp || (J.ny == G.ny && J.line != G.line)) continue;
-        for (unsigned a = 0; a < m.na; ++a)
-            for (unsigned b = 0; b < m.nb; ++b) {
-                if (J.ny != G.ny && (J.ny == nP ? a : b) != J.line) continue;
-                over[tr ? (size_t)b * m.na + a : (size_t)a * m.nb + b] |= (unsigned char)(1u << j);
-                any = true;
-            }
+        all.resize(at + (size_t)m.na * m.nb, 0);
+        unsigned a0 = 0, a1 = m.na, b0 = 0, b1 = m.nb;      // where face j meets this one
+        if (J.ny == nP) {
+            a0 = J.line;
+            a1 = J.line + 1;
+        } else if (J.ny == nPP) {
+            b0 = J.line;
+            b1 = J.line + 1;
+        }
+        for (unsigned a = a0; a < a1; ++a)
+            for (unsigned b = b0; b < b1; ++b)
+                all[at + (tr ? (size_t)b * m.na + a : (size_t)a * m.nb + b)] |= (unsigned char)(1u << j);
     }
-    if (!any) return 0;
-    unsigned char* d;
-    int rc = upload(h, &d, over.data(), over.size());
-    *out = d;
-    return rc;
+    return all.size() == at ? -1 : (long)at;
 }
 
 static int setup_hooks(ems_engine* h)
@@ -4535,13 +5230,19 @@ static int setup_hooks(ems_engine* h)
     };
     const int nmur = (int)h->mur.size();
     auto folded = [&](int k) { return k == h->mur_fold[0] || k == h->mur_fold[1]; };
-    auto mur_apply = [&](int k, HookPlan& q) {
-        q = mur_job(kMurApply, k);
-        for (int j = 0; j < nmur && j < (int)kMurMaskFaces; ++j) q.d.start[j] = h->mur[j].start_ts;
-        int rc = mur_over(h, k, 0, &q.d.over[0]);
-        return rc ? rc : mur_over(h, k, 1, &q.d.over[1]);
-    };
     int rc;
+    std::vector<unsigned char> over;
+    std::vector<long> over_at;
+    for (int k = 0; k < nmur; ++k)
+        for (int c = 0; c < 2; ++c) over_at.push_back(mur_over(h, k, c, over));
+    unsigned char* d_over = nullptr;
+    if (!over.empty() && (rc = upload(h, &d_over, over.data(), over.size()))) return rc;
+    auto mur_apply = [&](int k) {
+        HookPlan q = mur_job(kMurApply, k);
+        for (int j = 0; j < nmur && j < (int)kMurMaskFaces; ++j) q.d.start[j] = h->mur[j].start_ts;
+        for (int c = 0; c < 2; ++c) q.d.over[c] = over_at[2 * k + c] < 0 ? nullptr : d_over + over_at[2 * k + c];
+        return q;
+    };
     std::vector<HookPlan> pre, v, c;
     // before the voltage update: nothing here sets a field element, and the
     // current side's ADE reads currents that no hook sets before the current update
@@ -4572,8 +5273,7 @@ static int setup_hooks(ems_engine* h)
         for (int k = nmur - 1; k >= 0; --k)
             if (!folded(k)) v.push_back(mur_job(kMurPost, k));
         for (int k = nmur - 1; k >= 0; --k) {
-            HookPlan q;
-            if ((rc = mur_apply(k, q))) return rc;
+            HookPlan q = mur_apply(k);
             const int side = k == h->mur_fold[0] ? 0 : k == h->mur_fold[1] ? 1 : -1;
             if (side >= 0) {
                 q.d.list = h->mur_rim[side];
@@ -4641,9 +5341,7 @@ static int setup_hooks(ems_engine* h)
     std::vector<HookPlan> post, apply;
     for (int k = nmur - 1; k >= 0; --k) {
         post.push_back(mur_job(kMurPost, k));
-        HookPlan q;
-        if ((rc = mur_apply(k, q))) return rc;
-        apply.push_back(q);
+        apply.push_back(mur_apply(k));
     }
     // post and apply as one job where that changes no value read
     bool joint = nmur > 0;
@@ -4698,6 +5396,19 @@ int ems_get_quad(const ems_engine* h, int* on, unsigned* zdepth)
     return 0;
 }
 
+int ems_get_pair(const ems_engine* h, int* on, unsigned tile[3], unsigned* launches)
+{
+    if (!h) return fail(EMS_E_ARG, "null handle");
+    if (on) *on = h->pair ? 1 : 0;
+    if (tile) {
+        tile[0] = h->pair ? h->pargs.tx : 0;
+        tile[1] = h->pair ? h->pargs.ty : 0;
+        tile[2] = h->pair ? h->pargs.zd : 0;
+    }
+    if (launches) *launches = h->pair_launches;
+    return 0;
+}
+
 int ems_init(ems_engine* h)
 {
     if (!h) return fail(EMS_E_ARG, "null handle");
@@ -4708,6 +5419,7 @@ int ems_init(ems_engine* h)
     if ((rc = setup_fused(h))) return rc;
     if ((rc = setup_quad(h))) return rc;
     if ((rc = setup_vsrc(h))) return rc;
+    if ((rc = setup_pair(h))) return rc;
     if ((rc = setup_hooks(h))) return rc;
     // small compressed tables (both half steps' within 32 KiB) go to LDS in the quad kernels
     h->lds_tab = h->cmp && (size_t)4 * h->n_unique * sizeof(float4) <= kLdsTabBytes;
@@ -5261,6 +5973,40 @@ static int launch_step(ems_engine* h, hipEvent_t* ev)
     return 0;
 }
 
+// state n+2 written by k_pair becomes the current state
+static void swap_pair_buffers(ems_engine* h)
+{
+    swap_step_buffers(h);
+    std::swap(h->numts_dev, h->numts_alt);
+}
+
+// the next one or two of at most `left` timesteps, and their samples: two in
+// one launch where nothing samples the state between them; ev: the events of
+// the step's (or, for a pair, its first step's) kernels
+static int advance(ems_engine* h, unsigned left, hipEvent_t* ev, unsigned* done)
+{
+    int rc;
+    bool two = h->pair && left >= 2 && !probe_due(h, h->numTS + 1);
+    for (size_t k = 0; k < h->dumps.size() && two; ++k) {
+        unsigned ks;
+        two = !dump_sample(h->dumps[k], h->numTS + 1, &ks);
+    }
+    *done = two ? 2 : 1;
+    if (two) {
+        PairBufs B{h->V, h->I, h->pmlV.flux_in, h->pmlI.flux_in, h->V_alt, h->I_alt, h->flux_alt[0], h->flux_alt[1],
+                   h->numts_dev, h->numts_alt};
+        void* args[] = {&h->pargs, &B};
+        if (ev) (void)hipEventRecord(ev[0], h->stream);
+        HIPCHK(hipLaunchKernel(pair_kernel(h, h->pair_lds > kPairLds * sizeof(float) * h->pair_threads), dim3(h->pair_blocks),
+                               dim3(h->pair_threads), args, h->pair_lds, h->stream));
+        if (ev) (void)hipEventRecord(ev[1], h->stream);
+        swap_pair_buffers(h);
+        ++h->pair_launches;
+    } else if ((rc = launch_step(h, ev))) return rc;
+    h->numTS += *done;
+    return launch_samples(h);
+}
+
 int ems_set_profiling(ems_engine* h, int enable)
 {
     if (!h) return fail(EMS_E_ARG, "null handle");
@@ -5296,7 +6042,8 @@ static unsigned graph_steps(const ems_engine* h)
 static std::vector<unsigned char> chunk_key(const ems_engine* h, unsigned steps)
 {
     std::vector<unsigned char> key;
-    key.push_back((unsigned char)(h->fused && h->V != h->V_base ? 1 : 0));
+    key.push_back((unsigned char)(((h->fused || h->pair) && h->V != h->V_base ? 1 : 0) |
+                                  (h->pair && h->numts_dev > h->numts_alt ? 2 : 0)));
     for (unsigned k = 0; k < steps; ++k) {
         const unsigned ts = h->numTS + k;          // numTS before step k of the chunk
         unsigned char b = 0;
@@ -5327,19 +6074,17 @@ static int graph_chunk(ems_engine* h, unsigned steps)
     if (G) {
         HIPCHK(hipGraphLaunch(G->exec, h->stream));
         // host state as the captured launches left it
-        for (unsigned k = 0; k < steps; ++k) {
-            if (h->fused) swap_step_buffers(h);
-            ++h->numTS;
-        }
+        for (unsigned k = 2 * G->pairs; k < steps && h->fused; ++k) swap_step_buffers(h);
+        if (G->pairs & 1u) swap_pair_buffers(h);
+        h->pair_launches += G->pairs;
+        h->numTS += steps;
         ++h->graph_replays;
         return 0;
     }
     if (h->graphs.size() >= kMaxGraphs) {
         // too many distinct patterns: direct launches
-        for (unsigned k = 0; k < steps; ++k) {
-            int rc = launch_step(h, nullptr);
-            ++h->numTS;
-            if (!rc) rc = launch_samples(h);
+        for (unsigned k = 0, n; k < steps; k += n) {
+            int rc = advance(h, steps - k, nullptr, &n);
             if (rc) return rc;
         }
         return 0;
@@ -5348,11 +6093,9 @@ static int graph_chunk(ems_engine* h, unsigned steps)
     e.key = key;
     HIPCHK(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
     int lrc = 0;
-    for (unsigned k = 0; k < steps; ++k) {
-        if (!lrc) lrc = launch_step(h, nullptr);
-        ++h->numTS;
-        if (!lrc) lrc = launch_samples(h);
-    }
+    const unsigned pairs0 = h->pair_launches;
+    for (unsigned k = 0, n; k < steps && !lrc; k += n) lrc = advance(h, steps - k, nullptr, &n);
+    e.pairs = h->pair_launches - pairs0;
     const hipError_t ec = hipStreamEndCapture(h->stream, &e.graph);
     if (lrc) {
         if (ec == hipSuccess && e.graph) (void)hipGraphDestroy(e.graph);
@@ -5417,11 +6160,11 @@ int ems_iterate(ems_engine* h, unsigned nsteps)
     }
     HIPCHK(hipEventRecord(h->ev0, h->stream));
     unsigned s = 0;
-    for (; s < nprof; ++s) {
-        rc = launch_step(h, &h->kev[4 * (size_t)s]);
-        ++h->numTS;
-        if (!rc) rc = launch_samples(h);
-        if (rc) return rc;
+    // step of the events' first four, and whether that launch held two steps
+    std::vector<unsigned char> pairs(nprof, 0);
+    for (unsigned n; s < nprof; s += n) {
+        if ((rc = advance(h, nprof - s, &h->kev[4 * (size_t)s], &n))) return rc;
+        pairs[s] = n == 2;
     }
     if (h->graph_chunk) {
         const unsigned steps = graph_steps(h);
@@ -5435,12 +6178,8 @@ int ems_iterate(ems_engine* h, unsigned nsteps)
             s += steps;
         }
     }
-    for (; s < nsteps; ++s) {
-        rc = launch_step(h, nullptr);
-        ++h->numTS;
-        if (!rc) rc = launch_samples(h);
-        if (rc) return rc;
-    }
+    for (unsigned n; s < nsteps; s += n)
+        if ((rc = advance(h, nsteps - s, nullptr, &n))) return rc;
     HIPCHK(hipGetLastError());
     HIPCHK(hipEventRecord(h->ev1, h->stream));
     if (!h->async || nprof) {
@@ -5450,16 +6189,25 @@ int ems_iterate(ems_engine* h, unsigned nsteps)
         h->last_ms = ms;
     }
     if (nprof) {
-        double vsum = 0, csum = 0;
+        double vsum = 0, csum = 0, psum = 0;
+        unsigned np = 0;
         for (unsigned s = 0; s < nprof; ++s) {
             float a = 0, b = 0;
             HIPCHK(hipEventElapsedTime(&a, h->kev[4 * (size_t)s], h->kev[4 * (size_t)s + 1]));
-            HIPCHK(hipEventElapsedTime(&b, h->kev[4 * (size_t)s + 2], h->kev[4 * (size_t)s + 3]));
+            if (pairs[s]) {
+                psum += a;
+                ++np;
+                ++s;
+                continue;
+            }
             vsum += a;
+            HIPCHK(hipEventElapsedTime(&b, h->kev[4 * (size_t)s + 2], h->kev[4 * (size_t)s + 3]));
             csum += b;
         }
-        h->last_volt_ms = vsum / nprof;
-        h->last_curr_ms = csum / nprof;
+        // with pairs: their launches' average, and no current half step beside them
+        const unsigned one = nprof - 2 * np;
+        h->last_volt_ms = np ? psum / np : vsum / one;
+        h->last_curr_ms = np ? 0.0 : csum / one;
     }
     return 0;
 }

@@ -286,6 +286,13 @@ class EngineHIP:
         check(lib().ems_get_quad(self.h, C.byref(q), C.byref(d)))
         return q.value, d.value
 
+    def pair(self):
+        """(1 when two timesteps run per launch, else 0; tile columns x, y and planes; pairs advanced)"""
+        on, n = C.c_int(), C.c_uint()
+        t = (C.c_uint * 3)()
+        check(lib().ems_get_pair(self.h, C.byref(on), t, C.byref(n)))
+        return on.value, tuple(t), n.value
+
     def last_timing(self):
         t, v, c = C.c_double(), C.c_double(), C.c_double()
         check(lib().ems_last_timing(self.h, C.byref(t), C.byref(v), C.byref(c)))

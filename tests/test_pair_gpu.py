@@ -1,0 +1,129 @@
+"""Two timesteps per launch (k_pair) against the oracle and against the two
+half steps, bit for bit: tiles whose rims and last, partly filled tiles fall
+anywhere, chunks down to one plane, sources (voltage and current) on rims and
+chunk ends, UPML in both layouts with slab faces inside tiles and hook-only
+cells from random fields, both coefficient layouts, odd step counts, samples
+that force single steps between pairs, and graph replays of either parity."""
+import numpy as np
+import pytest
+
+from oracle.operator_ref import RefOperator
+from oracle.oracle import RefEngine
+from openems_amd import scenes
+from openems_amd.engine import EngineHIP
+from openems_amd.operator import Operator
+from openems_amd.simulation import Simulation
+
+pytestmark = pytest.mark.gpu
+
+
+def _cavity(nx, ny, nz, curr=False):
+    s = scenes.pec_cavity(8, 100)
+    s["lines"] = [np.arange(n, dtype=np.float64) for n in (nx, ny, nz)]
+    a = (nx // 2, ny // 2, nz // 2)
+    s["excitations"] = [{"type": 0, "val": (0.5, 0.0, 1.0), "start": a, "stop": (a[0] + 1, a[1], a[2] + 1)}]
+    if curr:
+        s["excitations"].append({"type": 2, "val": (0.0, 1.0, 0.3), "start": (2.5, 1.5, 1.5), "stop": (2.5, 2.5, 2.5)})
+    s["probes"] = []
+    return s
+
+
+def _graded(n, pml):
+    return scenes.upml_bricks(n, 100, nbricks=6, pml=pml, dump=False)
+
+
+def _sheet(nx, ny, nz):
+    """a source in every column of a plane, mesh edges included"""
+    s = _cavity(nx, ny, nz)
+    s["excitations"] = [{"type": 0, "val": (1.0, 0.5, 0.0), "start": (0, 0, nz // 2), "stop": (nx - 1, ny - 1, nz // 2)}]
+    return s
+
+
+CASES = [
+    # scene, tile (columns x, y, planes; None: the automatic one), layout, steps
+    ("cavity_5x4x3", lambda: _cavity(5, 4, 3), None, "auto", 9),
+    ("cavity_23x17x9_current_source", lambda: _cavity(23, 17, 9, True), "7,6,1", "auto", 21),
+    ("cavity_23x17x9_plain", lambda: _cavity(23, 17, 9, True), "10,6,4", "plain", 20),
+    ("cavity_66x34x12", lambda: _cavity(66, 34, 12), "64,16,5", "auto", 20),
+    ("cavity_64", lambda: _cavity(64, 64, 64), None, "auto", 41),
+    ("sheet_40x26x18", lambda: _sheet(40, 26, 18), "13,8,3", "auto", 30),
+    ("upml_40", lambda: _graded(40, 8), "16,12,7", "compressed", 60),
+    ("upml_40_plain", lambda: _graded(40, 8), "16,12,7", "plain", 61),
+    ("upml_45_pml6", lambda: _graded(45, 6), None, "compressed", 60),
+    ("upml_40_pml6_one_plane", lambda: _graded(40, 6), "40,9,1", "compressed", 40),
+    ("wires_36", lambda: scenes.wire_antenna(36, 100), "11,36,36", "auto", 80),
+]
+
+
+@pytest.mark.parametrize("name,make,tile,layout,steps", CASES, ids=[c[0] for c in CASES])
+def test_pairs_match_oracle_and_halves(gpu, monkeypatch, name, make, tile, layout, steps):
+    monkeypatch.setenv("EMS_PAIR", "1")
+    if tile:
+        monkeypatch.setenv("EMS_PAIR_TILE", tile)
+    scene = make()
+    print("case pairs", name, tile, layout, "steps", steps, flush=True)
+    op = Operator(scene)
+    eng = EngineHIP(op, layout=layout)
+    assert eng.pair()[0] == 1
+    eng.IterateTS(steps)
+    assert eng.pair()[2] == steps // 2
+    ref = RefEngine(RefOperator(scene).build(), "basic")
+    ref.iterate(steps)
+    rv, rc = ref.raw_views()
+    assert np.max(np.abs(rv)) > 0
+    assert np.array_equal(eng.get_volt(), rv)
+    assert np.array_equal(eng.get_curr(), rc)
+    ref.close()
+    # from random fields in every cell, the last lines included
+    rng = np.random.default_rng(5)
+    v = rng.standard_normal((3,) + tuple(op.N)).astype(np.float32)
+    c = rng.standard_normal((3,) + tuple(op.N)).astype(np.float32)
+    half = EngineHIP(op, layout=layout, fused=False)
+    assert half.pair()[0] == 0
+    half.IterateTS(steps)
+    for e in (eng, half):
+        e.set_volt(v)
+        e.set_curr(c)
+        e.IterateTS(steps)
+    assert np.array_equal(eng.get_volt(), half.get_volt())
+    assert np.array_equal(eng.get_curr(), half.get_curr())
+    eng.close()
+    half.close()
+
+
+@pytest.mark.parametrize("n,graph", [(40, 0), (40, 24), (64, 7)])
+def test_pairs_with_samples_and_graphs(gpu, monkeypatch, n, graph):
+    """Probes and dumps fall on odd and even steps: their steps run singly
+    where needed; replayed chunks equal direct launches and the half steps."""
+    monkeypatch.setenv("EMS_PAIR", "1")
+    scene = scenes.upml_bricks(n, 700, nbricks=4) if n == 40 else scenes.pec_cavity(n, 700)
+    print("case pairs with samples", n, "graph", graph, flush=True)
+    out = []
+    for fused in (None, False):
+        sim = Simulation(scene, fused=fused, graph=graph)
+        sim.run(301)
+        sim.run(3)
+        sim.run(396)
+        assert (sim.eng.pair()[2] > 100) == (fused is None)
+        out.append((sim.results(), sim.eng.get_volt(), sim.eng.get_curr(), sim.eng.energy()))
+        sim.close()
+    (ra, va, ca, ea), (rb, vb, cb, eb) = out
+    for k in rb["probes"]:
+        assert np.array_equal(ra["probes"][k]["td"], rb["probes"][k]["td"])
+    for k in rb["dumps"]:
+        assert np.array_equal(ra["dumps"][k]["fd"], rb["dumps"][k]["fd"])
+    assert np.array_equal(va, vb) and np.array_equal(ca, cb) and ea == eb
+
+
+def test_pair_policy(gpu, monkeypatch):
+    """Automatic engines without hooks between the half steps take pairs, UPML
+    meshes from a million cells on; asked-for step forms and lane widths do not."""
+    monkeypatch.delenv("EMS_PAIR", raising=False)
+    small, pml = Operator(_cavity(24, 20, 16)), Operator(_graded(40, 6))
+    for op, kw, want in ((small, {}, 1), (small, {"fused": False}, 0), (small, {"quad": True}, 0), (small, {"quad": False}, 0),
+                         (small, {"fused": "lds"}, 0), (pml, {}, 0),
+                         (Operator(scenes.mur_layers(24, 20, 16, 10)), {}, 0), (Operator(scenes.dispersive_rlc(40, 10)), {}, 0),
+                         (Operator(_cavity(260, 12, 10)), {}, 1)):
+        eng = EngineHIP(op, **kw)
+        assert eng.pair()[0] == want, (op.N, kw)
+        eng.close()
