@@ -67,3 +67,28 @@ def test_hooks_match_oracle(gpu, name, make, steady):
     assert np.array_equal(eng.get_curr(), rc)
     eng.close()
     e.close()
+
+
+@pytest.mark.parametrize("nprobe", [1, 191, 400])
+def test_steady_state_of_many_probes(gpu, nprobe):
+    """More probes than the evaluation has threads, and one."""
+    scene = _layers([2] * 6)
+    op = Operator(scene)
+    period, _, _ = steady_state_probes(op)
+    rng = np.random.default_rng(nprobe)
+    dirs = rng.integers(0, 3, nprobe).tolist()
+    pos = [[int(rng.integers(0, k)) for k in op.N] for _ in range(nprobe)]
+    print("case steady state,", nprobe, "probes", flush=True)
+    eng = EngineHIP(op, fused=False, steady_state=(period, dirs, pos))
+    eng.IterateTS(6 * period + 3)
+    ref = RefEngine(RefOperator(scene).build(), "basic", steady_state=(period, dirs, pos))
+    ref.iterate(6 * period + 3)
+    last, hist = eng.steady_state()
+    want = ref.steady_history()
+    assert len(hist) == len(want) and len(want) > 3 and last == hist[-1][1]
+    for (t1, d1), (t2, d2) in zip(hist, want):
+        assert t1 == t2
+        # the energy is summed in another order than the oracle's
+        assert d1 == pytest.approx(d2, rel=1e-9, abs=1e-300)
+    eng.close()
+    ref.close()
