@@ -3300,15 +3300,49 @@ __device__ __forceinline__ void pml_coefs(const PmlArgs& P, unsigned long long l
     }
 }
 
+// objective probes: F_p += (V[lin_p] / div_p) * w, w = exp(-2 pi i f t) * dT
+// at t = ts*dT (voltages after step ts)
+struct AdjProbe {
+    unsigned long long lin;
+    double div;
+};
+
+// adjoint source of J = sum |F_p|^2 at step ts: dJ/dV = 2 Re(conj(F) w) / div
+struct AdjSrc {
+    float* lV;
+    const AdjProbe* pr;
+    unsigned np;
+    double f, dT;
+    unsigned ts;
+    const double* F;
+};
+
+__device__ __forceinline__ void adj_source(const AdjSrc& s, unsigned p)
+{
+    if (p >= s.np) return;
+    const double t = (double)s.ts * s.dT;
+    const double ph = -2.0 * 3.141592653589793238462643383279 * s.f * t;
+    const double g = 2.0 * (s.F[2 * p] * cos(ph) * s.dT + s.F[2 * p + 1] * sin(ph) * s.dT) / s.pr[p].div;
+    s.lV[s.pr[p].lin] = (float)((double)s.lV[s.pr[p].lin] + g);
+}
+
 // transposed current half step, one thread per (x, y) column sweeping z.
 // lI' = lI + curl_I^T(B) (B: curl adjoint left by the transposed voltage
 // half step of the later timestep); writes lI, lFI and A = curl_V adjoint.
+// The workgroups past the mesh's add the adjoint source of this step's
+// objective to the voltages' adjoint, which this half step does not touch (a
+// launch of its own took 3.2 us of 31).
 template <int PM, bool CC>
 __global__ __launch_bounds__(kBlock) void k_adj_curr(const GridDesc g, float* __restrict__ lI,
                                                      const float* __restrict__ B, float* __restrict__ A,
-                                                     const CoefArgs k, const PmlArgs pml, float* __restrict__ lFI)
+                                                     const CoefArgs k, const PmlArgs pml, float* __restrict__ lFI,
+                                                     unsigned nblk, const AdjSrc src)
 {
-    const unsigned t = xcd_tile(blockIdx.x, gridDim.x);
+    if (blockIdx.x >= nblk) {
+        adj_source(src, (blockIdx.x - nblk) * kBlock + threadIdx.x);
+        return;
+    }
+    const unsigned t = xcd_tile(blockIdx.x, nblk);
     const unsigned qt = t % g.qtiles, zc = t / g.qtiles;
     unsigned x, y;
     if (!tile_column(g, qt, x, y)) return;
@@ -3316,6 +3350,7 @@ __global__ __launch_bounds__(kBlock) void k_adj_curr(const GridDesc g, float* __
     const unsigned long long cs = g.cs;
     const unsigned Nx = g.Nx;
     const bool col_upd = x + 1 < g.Nx && y + 1 < g.Ny;
+    const unsigned pcm = PM != kNoPml ? pml_colmask(pml, (int)x, (int)y) : 0u;
     for (unsigned z = z0; z < z1; ++z) {
         const unsigned long long p = x + (unsigned long long)Nx * y + (unsigned long long)g.plane * z;
         // lI' = lI + curl_I^T(B); curl_I of the voltage update uses lower
@@ -3338,8 +3373,8 @@ __global__ __launch_bounds__(kBlock) void k_adj_curr(const GridDesc g, float* __
         }
         const bool upd = col_upd && z + 1 < g.Nz;
         float lo[3], a[3] = {0.0f, 0.0f, 0.0f};
-        unsigned long long li = 0;
-        const bool in_pml = PM != kNoPml && pml_at(pml, (int)x, (int)y, (int)z, li);
+        unsigned li = 0;
+        const bool in_pml = PM != kNoPml && pcm && pml_at_col(pml, pcm, (int)x, (int)y, (int)z, li);
         if (upd) {
             float ca[3], cb[3];
             load_coef<CC>(k, cs, p, CC ? k.idx[p] : 0u, ca, cb);
@@ -3399,6 +3434,7 @@ __global__ __launch_bounds__(kBlock) void k_adj_volt(const GridDesc g, float* __
     const unsigned z0 = zc * g.zdepth, z1 = min(z0 + g.zdepth, g.Nz);
     const unsigned long long cs = g.cs;
     const unsigned Nx = g.Nx;
+    const unsigned pcm = PM != kNoPml ? pml_colmask(pml, (int)x, (int)y) : 0u;
     for (unsigned z = z0; z < z1; ++z) {
         const unsigned long long p = x + (unsigned long long)Nx * y + (unsigned long long)g.plane * z;
         // lV' = lV + curl_V^T(A); curl_V of the current update uses upper
@@ -3420,8 +3456,8 @@ __global__ __launch_bounds__(kBlock) void k_adj_volt(const GridDesc g, float* __
         }
         float ca[3], cb[3], lo[3], b[3];
         load_coef<CC>(k, cs, p, CC ? k.idx[p] : 0u, ca, cb);
-        unsigned long long li = 0;
-        const bool in_pml = PM != kNoPml && pml_at(pml, (int)x, (int)y, (int)z, li);
+        unsigned li = 0;
+        const bool in_pml = PM != kNoPml && pcm && pml_at_col(pml, pcm, (int)x, (int)y, (int)z, li);
         if (in_pml) {
             float k0[3], ko[3], kn[3];
             pml_coefs<PM>(pml, li, k0, ko, kn);
@@ -3455,12 +3491,27 @@ __global__ __launch_bounds__(kBlock) void k_adj_volt(const GridDesc g, float* __
     }
 }
 
-// forward curl of the currents and the voltages on the box edges before a
-// step (the inputs of the coming voltage update)
-__global__ void k_adj_record(const GridDesc g, const float* __restrict__ V, const float* __restrict__ I,
-                             const AdjBox box, float* __restrict__ hc, float* __restrict__ hv)
+// After a forward step (and before the first): the running DFT of the
+// objective probes (last workgroups, np = 0 before the first step) and, where
+// hc is given, the forward curl of the currents and the voltages on the box
+// edges, the inputs of the coming voltage update.
+__global__ __launch_bounds__(kBlock) void k_adj_sample(const GridDesc g, const float* __restrict__ V,
+                                                       const float* __restrict__ I, const AdjBox box,
+                                                       float* __restrict__ hc, float* __restrict__ hv, unsigned rblk,
+                                                       const AdjProbe* __restrict__ pr, unsigned np, double f, double dT,
+                                                       const unsigned* __restrict__ numts, double* __restrict__ F)
 {
-    const unsigned long long kk = blockIdx.x * (unsigned long long)blockDim.x + threadIdx.x;
+    if (blockIdx.x >= rblk) {
+        const unsigned q = (blockIdx.x - rblk) * kBlock + threadIdx.x;
+        if (q >= np) return;
+        const double t = (double)*numts * dT;
+        const double ph = -2.0 * 3.141592653589793238462643383279 * f * t;
+        const double v = (double)V[pr[q].lin] / pr[q].div;
+        F[2 * q] += v * cos(ph) * dT;
+        F[2 * q + 1] += v * sin(ph) * dT;
+        return;
+    }
+    const unsigned long long kk = blockIdx.x * (unsigned long long)kBlock + threadIdx.x;
     if (kk >= box.n) return;
     const unsigned x = box.x0 + (unsigned)(kk % box.nx);
     const unsigned y = box.y0 + (unsigned)((kk / box.nx) % box.ny);
@@ -3476,37 +3527,6 @@ __global__ void k_adj_record(const GridDesc g, const float* __restrict__ V, cons
     hc[2 * box.n + kk] = Iy[p] - Iy[p - xm] - Ix[p] + Ix[p - ym];
 #pragma unroll
     for (int n = 0; n < 3; ++n) hv[n * box.n + kk] = V[n * cs + p];
-}
-
-// objective probes: F_p += (V[lin_p] / div_p) * w, w = exp(-2 pi i f t) * dT
-// at t = ts*dT (voltages after step ts)
-struct AdjProbe {
-    unsigned long long lin;
-    double div;
-};
-
-__global__ void k_adj_dft(const float* __restrict__ V, const AdjProbe* __restrict__ pr, unsigned np, double f,
-                          double dT, const unsigned* __restrict__ numts, double* __restrict__ F)
-{
-    const unsigned p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= np) return;
-    const double t = (double)*numts * dT;
-    const double ph = -2.0 * 3.141592653589793238462643383279 * f * t;
-    const double v = (double)V[pr[p].lin] / pr[p].div;
-    F[2 * p] += v * cos(ph) * dT;
-    F[2 * p + 1] += v * sin(ph) * dT;
-}
-
-// adjoint source of J = sum |F_p|^2 at step ts: dJ/dV = 2 Re(conj(F) w) / div
-__global__ void k_adj_src(float* __restrict__ lV, const AdjProbe* __restrict__ pr, unsigned np, double f, double dT,
-                          unsigned ts, const double* __restrict__ F)
-{
-    const unsigned p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= np) return;
-    const double t = (double)ts * dT;
-    const double ph = -2.0 * 3.141592653589793238462643383279 * f * t;
-    const double g = 2.0 * (F[2 * p] * cos(ph) * dT + F[2 * p + 1] * sin(ph) * dT) / pr[p].div;
-    lV[pr[p].lin] = (float)((double)lV[pr[p].lin] + g);
 }
 
 // ---------------------------------------------------------------------------
@@ -7241,7 +7261,11 @@ struct ems_adjoint {
     std::vector<double> F;
     std::vector<AdjCkpt> ck;   // state at n0 + s*K, s = 0..S-1, then the final state
     float *lV = nullptr, *lI = nullptr, *A = nullptr, *B = nullptr, *lFV = nullptr, *lFI = nullptr;
-    float *hc = nullptr, *hv = nullptr;   // [K][3][box.n]
+    // recorded inputs of the voltage updates, [rec_steps][3][box.n] each: of
+    // every forward step where they fit (kept), else of one segment
+    float *hc = nullptr, *hv = nullptr;
+    size_t rec_steps = 0;
+    bool kept = false;
     double *gvi = nullptr, *gvv = nullptr;
     bool forward_done = false;
     std::vector<void*> allocs;
@@ -7300,30 +7324,79 @@ int adj_restore(ems_adjoint* a, const AdjCkpt& c)
     return 0;
 }
 
+// Records of every forward step, or of one segment.  Kept, they save the
+// reverse pass its replay of the forward steps (a third of it): the box is a
+// small part of the mesh (17 x 17 x 7 edges: 48 KB a step), so they stay
+// wherever they take at most an eighth of the free memory; beyond that the
+// states saved every K steps are replayed.  EMS_ADJ_KEEP=0 always replays.
+int adj_reserve(ems_adjoint* a, unsigned nsteps)
+{
+    const size_t step = 3 * a->box.n * sizeof(float);
+    auto release = [&] {
+        if (a->hc) (void)hipFree(a->hc);
+        if (a->hv) (void)hipFree(a->hv);
+        a->hc = a->hv = nullptr;
+        a->rec_steps = 0;
+    };
+    auto grow = [&](size_t n) {
+        if (a->rec_steps >= n) return true;
+        release();
+        if (hipMalloc((void**)&a->hc, n * step) != hipSuccess || hipMalloc((void**)&a->hv, n * step) != hipSuccess) {
+            (void)hipGetLastError();
+            release();
+            return false;
+        }
+        a->rec_steps = n;
+        return true;
+    };
+    size_t freeb = 0, totalb = 0;
+    bool keep = true;
+    if (const char* e = std::getenv("EMS_ADJ_KEEP")) keep = std::atoi(e) != 0;
+    if (a->rec_steps < nsteps)
+        keep = keep && hipMemGetInfo(&freeb, &totalb) == hipSuccess && 2 * (unsigned long long)nsteps * step <= freeb / 8;
+    a->kept = keep && grow(nsteps);
+    if (!a->kept && !grow(std::min(a->K, nsteps))) return fail(EMS_E_NOMEM, "no device memory for the adjoint's records");
+    return 0;
+}
+
+// the record of step `rec` (-1: none) and, after a forward step, the running DFT
+void adj_sample(ems_adjoint* a, int rec, bool dft)
+{
+    ems_engine* h = a->h;
+    const unsigned rblk = rec < 0 ? 0 : (unsigned)((a->box.n + kBlock - 1) / kBlock);
+    const unsigned np = dft ? a->np : 0, nb = rblk + (np + kBlock - 1) / kBlock;
+    const size_t at = rec < 0 ? 0 : (size_t)rec * 3 * a->box.n;
+    if (nb)
+        hipLaunchKernelGGL(k_adj_sample, dim3(nb), dim3(kBlock), 0, h->stream, h->g, h->V, h->I, a->box, a->hc + at,
+                           a->hv + at, rblk, a->d_probes, np, a->freq, a->dT, h->numts_dev, a->d_F);
+}
+
 template <int PM, bool CC>
-void adj_kernels_t(ems_adjoint* a, const float* hc, const float* hv)
+void adj_kernels_t(ems_adjoint* a, const float* hc, const float* hv, unsigned ts)
 {
     ems_engine* h = a->h;
     const unsigned nblk = h->g.qtiles * h->g.nzc;
     PmlArgs pI = h->pmlI, pV = h->pmlV;
-    hipLaunchKernelGGL((k_adj_curr<PM, CC>), dim3(nblk), dim3(kBlock), 0, h->stream, h->g, a->lI, a->B, a->A, h->kI,
-                       pI, a->lFI);
+    hipLaunchKernelGGL((k_adj_curr<PM, CC>), dim3(nblk + (a->np + kBlock - 1) / kBlock), dim3(kBlock), 0, h->stream, h->g,
+                       a->lI, a->B, a->A, h->kI, pI, a->lFI, nblk,
+                       AdjSrc{a->lV, a->d_probes, a->np, a->freq, a->dT, ts, a->d_F});
     hipLaunchKernelGGL((k_adj_volt<PM, CC>), dim3(nblk), dim3(kBlock), 0, h->stream, h->g, a->lV, a->A, a->B, h->kV,
                        pV, a->lFV, a->box, hc, hv, a->gvi, a->gvv);
 }
 
-void adj_kernels(ems_adjoint* a, const float* hc, const float* hv)
+// one reverse step: the source of step ts, the transposed half steps
+void adj_kernels(ems_adjoint* a, const float* hc, const float* hv, unsigned ts)
 {
     ems_engine* h = a->h;
     const int pm = h->pmlV.n ? h->pml_mode : kNoPml;
     if (h->cmp) {
-        if (pm == kPmlCompressed) adj_kernels_t<kPmlCompressed, true>(a, hc, hv);
-        else if (pm == kPmlPlain) adj_kernels_t<kPmlPlain, true>(a, hc, hv);
-        else adj_kernels_t<kNoPml, true>(a, hc, hv);
+        if (pm == kPmlCompressed) adj_kernels_t<kPmlCompressed, true>(a, hc, hv, ts);
+        else if (pm == kPmlPlain) adj_kernels_t<kPmlPlain, true>(a, hc, hv, ts);
+        else adj_kernels_t<kNoPml, true>(a, hc, hv, ts);
     } else {
-        if (pm == kPmlCompressed) adj_kernels_t<kPmlCompressed, false>(a, hc, hv);
-        else if (pm == kPmlPlain) adj_kernels_t<kPmlPlain, false>(a, hc, hv);
-        else adj_kernels_t<kNoPml, false>(a, hc, hv);
+        if (pm == kPmlCompressed) adj_kernels_t<kPmlCompressed, false>(a, hc, hv, ts);
+        else if (pm == kPmlPlain) adj_kernels_t<kPmlPlain, false>(a, hc, hv, ts);
+        else adj_kernels_t<kNoPml, false>(a, hc, hv, ts);
     }
 }
 
@@ -7386,7 +7459,6 @@ int ems_adj_create(ems_adjoint** out, ems_engine* h, unsigned nprobe, const unsi
     if ((rc = a->alloc(&a->d_probes, nprobe)) || (rc = a->alloc(&a->d_F, 2 * nprobe)) || (rc = a->alloc(&a->lV, c3)) ||
         (rc = a->alloc(&a->lI, c3)) || (rc = a->alloc(&a->A, c3)) || (rc = a->alloc(&a->B, c3)) ||
         (rc = a->alloc(&a->lFV, f3V)) || (rc = a->alloc(&a->lFI, f3I)) ||
-        (rc = a->alloc(&a->hc, (size_t)a->K * 3 * box.n)) || (rc = a->alloc(&a->hv, (size_t)a->K * 3 * box.n)) ||
         (rc = a->alloc(&a->gvi, 3 * box.n)) || (rc = a->alloc(&a->gvv, 3 * box.n)))
         return bail(rc);
     if (hipMemcpy(a->d_probes, pr.data(), nprobe * sizeof(AdjProbe), hipMemcpyHostToDevice) != hipSuccess)
@@ -7409,16 +7481,19 @@ int ems_adj_forward(ems_adjoint* a, unsigned nsteps, double* J)
     a->nsteps = nsteps;
     const unsigned S = (nsteps + a->K - 1) / a->K;
     if (a->ck.size() < (size_t)S + 1) a->ck.resize(S + 1);
-    const unsigned T = 256;
+    if ((rc = adj_reserve(a, nsteps))) return rc;
+    // with every step's record kept, the reverse pass needs no replay and so
+    // no saved states on the way
+    if (a->kept) adj_sample(a, 0, false);
     for (unsigned s = 0; s < S; ++s) {
-        if ((rc = adj_save(a, a->ck[s]))) return rc;
+        if (!a->kept && (rc = adj_save(a, a->ck[s]))) return rc;
         const unsigned len = std::min(a->K, nsteps - s * a->K);
         for (unsigned j = 0; j < len; ++j) {
             rc = launch_step(h, nullptr);
             ++h->numTS;
             if (rc) return rc;
-            hipLaunchKernelGGL(k_adj_dft, dim3((a->np + T - 1) / T), dim3(T), 0, h->stream, h->V, a->d_probes, a->np,
-                               a->freq, a->dT, h->numts_dev, a->d_F);
+            const unsigned n = s * a->K + j + 1;
+            adj_sample(a, a->kept && n < nsteps ? (int)n : -1, true);
         }
     }
     if ((rc = adj_save(a, a->ck[S]))) return rc;
@@ -7452,26 +7527,24 @@ int ems_adj_backward(ems_adjoint* a, double* dJ_dvi, double* dJ_dvv)
     HIPCHK(hipMemsetAsync(a->gvi, 0, 3 * a->box.n * sizeof(double), h->stream));
     HIPCHK(hipMemsetAsync(a->gvv, 0, 3 * a->box.n * sizeof(double), h->stream));
     const unsigned S = (a->nsteps + a->K - 1) / a->K;
-    const unsigned T = 256;
-    const unsigned rblk = (unsigned)((a->box.n + T - 1) / T);
     int rc;
     for (int s = (int)S - 1; s >= 0; --s) {
-        if ((rc = adj_restore(a, a->ck[s]))) return rc;
         const unsigned len = std::min(a->K, a->nsteps - s * a->K);
-        // replay the segment, recording the inputs of each voltage update
-        for (unsigned j = 0; j < len; ++j) {
-            hipLaunchKernelGGL(k_adj_record, dim3(rblk), dim3(T), 0, h->stream, h->g, h->V, h->I, a->box,
-                               a->hc + (size_t)j * 3 * a->box.n, a->hv + (size_t)j * 3 * a->box.n);
-            rc = launch_step(h, nullptr);
-            ++h->numTS;
-            if (rc) return rc;
+        const size_t first = a->kept ? (size_t)s * a->K : 0;      // record of the segment's first step
+        if (!a->kept) {
+            // replay the segment, recording the inputs of each voltage update
+            if ((rc = adj_restore(a, a->ck[s]))) return rc;
+            for (unsigned j = 0; j < len; ++j) {
+                adj_sample(a, (int)j, false);
+                rc = launch_step(h, nullptr);
+                ++h->numTS;
+                if (rc) return rc;
+            }
         }
         // reverse steps of the segment
         for (int j = (int)len - 1; j >= 0; --j) {
-            const unsigned ts = a->n0 + (unsigned)s * a->K + (unsigned)j + 1;
-            hipLaunchKernelGGL(k_adj_src, dim3((a->np + T - 1) / T), dim3(T), 0, h->stream, a->lV, a->d_probes,
-                               a->np, a->freq, a->dT, ts, a->d_F);
-            adj_kernels(a, a->hc + (size_t)j * 3 * a->box.n, a->hv + (size_t)j * 3 * a->box.n);
+            const size_t at = (first + (size_t)j) * 3 * a->box.n;
+            adj_kernels(a, a->hc + at, a->hv + at, a->n0 + (unsigned)s * a->K + (unsigned)j + 1);
         }
     }
     HIPCHK(hipGetLastError());
@@ -7490,6 +7563,8 @@ void ems_adj_destroy(ems_adjoint* a)
         if (a->h->stream) hipStreamSynchronize(a->h->stream);
     }
     for (void* p : a->allocs) hipFree(p);
+    if (a->hc) hipFree(a->hc);
+    if (a->hv) hipFree(a->hv);
     delete a;
 }
 

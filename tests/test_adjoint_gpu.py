@@ -179,3 +179,22 @@ def test_full_size_directional_derivative(gpu):
     print("J", J, "adjoint", ad, "fd", fd, flush=True)
     assert J > 0 and fd != 0
     assert abs(ad - fd) <= 1e-3 * abs(fd)
+
+
+@pytest.mark.parametrize("steps,every", [(1, 8), (37, 8), (64, 64)])
+def test_kept_records_equal_replayed_segments(gpu, monkeypatch, steps, every):
+    """The gradient from records kept during the forward run equals the one
+    from replayed segments bit for bit, also after a second, longer run, and
+    the engine ends at the same state."""
+    scene, probes, freq = _small()
+    eps = scene["materials"][0]["grid"]["eps"].copy()
+    out = []
+    for keep in ("1", "0"):
+        monkeypatch.setenv("EMS_ADJ_KEEP", keep)
+        print("case adjoint records, keep", keep, "steps", steps, flush=True)
+        prob = DesignProblem(scene, probes, freq, 200 + steps, checkpoint_every=every)
+        out.append(prob.value_and_grad(eps) + (prob._eng.get_volt(), prob._eng.get_curr(), prob._eng.numTS))
+        prob.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+    assert np.abs(out[0][1]).max() > 0
