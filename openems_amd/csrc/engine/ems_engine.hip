@@ -866,10 +866,11 @@ __global__ __launch_bounds__(kBlock) void k_volt4(const GridDesc g, const QBoxes
     }
 }
 
+// workgroup `bid` of the half step's `nblk`
 template <int PM, bool CC, bool NT, bool LT>
-__global__ __launch_bounds__(kBlock) void k_curr4(const GridDesc g, const QBoxes boxes, float* I,
-                                                  const float* __restrict__ V, const CoefArgs kg, const PmlArgs pml,
-                                                  unsigned* __restrict__ numts)
+__device__ __forceinline__ void curr4_tile(const GridDesc& g, const QBoxes& boxes, unsigned bid, unsigned nblk, float* I,
+                                           const float* __restrict__ V, const CoefArgs& kg, const PmlArgs& pml,
+                                           unsigned* __restrict__ numts)
 {
     extern __shared__ float4 s_tab[];
     CoefArgs k = kg;
@@ -879,9 +880,9 @@ __global__ __launch_bounds__(kBlock) void k_curr4(const GridDesc g, const QBoxes
         k.tab = s_tab;
     }
     unsigned x0, y, z0, z1;
-    const bool lane = qbox_cell(boxes, xcd_tile(blockIdx.x, gridDim.x), x0, y, z0, z1);
+    const bool lane = qbox_cell(boxes, xcd_tile(bid, nblk), x0, y, z0, z1);
     // one launch of the half step advances the timestep counter
-    if (numts && blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(numts, 1u);
+    if (numts && bid == 0 && threadIdx.x == 0) atomicAdd(numts, 1u);
     if (!lane) return;
     const bool yupd = y + 1 < g.Ny;
     // elements the main update covers along x (x < Nx-1)
@@ -956,6 +957,14 @@ __global__ __launch_bounds__(kBlock) void k_curr4(const GridDesc g, const QBoxes
             for (int n = 0; n < 3; ++n) st4<NT>(I + n * cs + p, out[n]);
         }
     }
+}
+
+template <int PM, bool CC, bool NT, bool LT>
+__global__ __launch_bounds__(kBlock) void k_curr4(const GridDesc g, const QBoxes boxes, float* I,
+                                                  const float* __restrict__ V, const CoefArgs kg, const PmlArgs pml,
+                                                  unsigned* __restrict__ numts)
+{
+    curr4_tile<PM, CC, NT, LT>(g, boxes, blockIdx.x, gridDim.x, I, V, kg, pml, numts);
 }
 
 // ---------------------------------------------------------------------------
@@ -2677,11 +2686,13 @@ struct SteadyDev {
 // (setup_hooks) keeps the reference's order and opens a new launch only where
 // a hook reads or writes a field element that an earlier hook of the launch
 // writes.  A workgroup belongs to one job (first[] in the kernel arguments).
-// Six Mur faces with steady-state detection (96 x 90 x 70): 22 -> 6 launches
-// and 66.0 -> 32.4 us per step; Drude, Lorentz and Debye boxes with RLC
-// elements (72^3): 17 -> 6 launches and 38.3 -> 23.0 us per step; one Mur
-// face (27 x 11 x 33): 6 -> 4 launches and 17.4 -> 15.3 us per step; 512 x
-// 384 x 320 layers around the quad sweep: 0.984 -> 0.959 ms per step.
+// With the hooks before an update beside other work (the currents' after the
+// voltage update, the voltages' beside the current update of the step before:
+// k_curr_pre), launches and time per step: six Mur faces with steady-state
+// detection (96 x 90 x 70) 22 -> 5 and 64.7 -> 26.9 us; Drude, Lorentz and
+// Debye boxes with RLC elements (72^3) 17 -> 4 and 38.2 -> 20.3 us; one Mur
+// face (27 x 11 x 33) 6 -> 3 and 17.3 -> 11.7 us; 512 x 384 x 320 layers
+// around the quad sweep, which has no such update, 0.984 -> 0.959 ms.
 //
 //   MurPre / MurPost / MurApply  Engine_Ext_Mur_ABC (engine_ext_mur_abc.cpp:68-178);
 //                  the faces' applies run in reverse creation order, so where
@@ -2745,22 +2756,24 @@ __device__ __forceinline__ bool mur_overset(const HookJob& J, int c, unsigned k,
     return o;
 }
 
-__global__ __launch_bounds__(kBlock) void k_hooks(float* __restrict__ V, float* __restrict__ I,
-                                                  const unsigned long long cs, const HookLaunch L,
-                                                  const unsigned* __restrict__ numts)
+// the job of the launch's workgroup `bid`, k: the thread within the job
+__device__ __forceinline__ const HookJob& hook_job(const HookLaunch& L, unsigned bid, unsigned& k)
 {
     unsigned w = 0, f = 0;
 #pragma unroll
     for (unsigned i = 1; i < kMaxHookJobs; ++i)
-        if (i < L.n && blockIdx.x >= L.first[i]) {
+        if (i < L.n && bid >= L.first[i]) {
             w = i;
             f = L.first[i];
         }
-    const HookJob& J = L.jobs[w];
-    unsigned k = (blockIdx.x - f) * kBlock + threadIdx.x;
-    if (k >= J.n) return;
-    const unsigned ts = *numts;
-    float* F = J.curr ? I : V;
+    k = (bid - f) * kBlock + threadIdx.x;
+    return L.jobs[w];
+}
+
+// the hooks before an update: they read F and set the extensions' own values
+__device__ __forceinline__ void hook_pre(const HookJob& J, unsigned k, const float* __restrict__ F,
+                                         const unsigned long long cs, unsigned ts)
+{
     switch (J.kind) {
     case kMurPre: {
         const MurDev& m = J.mur;
@@ -2770,6 +2783,43 @@ __global__ __launch_bounds__(kBlock) void k_hooks(float* __restrict__ V, float* 
         m.mPP[k] = F[m.offPP + s] - m.cPP[k] * F[m.offPP + p];
         return;
     }
+    case kRlcPre: {
+        const RlcDev& r = J.rlc;
+        const float* Vd1 = r.vd + rlc_slot(ts, 1) * r.count;
+        r.il[k] = r.il[k] + (r.c[0][k] * r.c[1][k]) * Vd1[k];
+        return;
+    }
+    case kLorPre: {                // k = component * count + cell
+        const LorDev& d = J.lor;
+        const unsigned n = k / d.count;
+        const float x = F[n * cs + d.lin[k - n * d.count]];
+        const float ade = d.ade[k] * d.cint[k];
+        if (d.clor) {
+            const float l = d.lor[k] + d.clor[k] * d.ade[k];
+            d.lor[k] = l;
+            d.ade[k] = ade + d.cext[k] * (x - l);
+        } else {
+            d.ade[k] = ade + d.cext[k] * x;
+        }
+        return;
+    }
+    }
+}
+
+// numts: [0] the counter, [1] the timestep of the pre hooks that run beside
+// the current update (k_curr_pre): that update advances [0], so the launch
+// between the two half steps leaves them the value it will have
+__global__ __launch_bounds__(kBlock) void k_hooks(float* __restrict__ V, float* __restrict__ I,
+                                                  const unsigned long long cs, const HookLaunch L,
+                                                  unsigned* __restrict__ numts)
+{
+    unsigned k;
+    const HookJob& J = hook_job(L, blockIdx.x, k);
+    const unsigned ts = numts[0];
+    if (blockIdx.x == 0 && threadIdx.x == 0) numts[1] = ts + 1u;
+    if (k >= J.n) return;
+    float* F = J.curr ? I : V;
+    switch (J.kind) {
     case kMurPost:
     case kMurPostApply: {
         const MurDev& m = J.mur;
@@ -2796,12 +2846,6 @@ __global__ __launch_bounds__(kBlock) void k_hooks(float* __restrict__ V, float* 
         if (!mur_overset(J, 1, k, ts)) F[m.offPP + p] = m.mPP[k];
         return;
     }
-    case kRlcPre: {
-        const RlcDev& r = J.rlc;
-        const float* Vd1 = r.vd + rlc_slot(ts, 1) * r.count;
-        r.il[k] = r.il[k] + (r.c[0][k] * r.c[1][k]) * Vd1[k];
-        return;
-    }
     case kRlcApply: {
         const RlcDev& r = J.rlc;
         float* V0 = r.vd + rlc_slot(ts, 0) * r.count;
@@ -2814,20 +2858,6 @@ __global__ __launch_bounds__(kBlock) void k_hooks(float* __restrict__ V, float* 
         V0[k] = v;
         J0[k] = r.c[6][k] * (v - V2[k]) - (r.c[7][k] * r.c[6][k]) * J1[k] - (r.c[8][k] * r.c[6][k]) * J2[k];
         F[r.lin[k]] = v;
-        return;
-    }
-    case kLorPre: {                // k = component * count + cell
-        const LorDev& d = J.lor;
-        const unsigned n = k / d.count;
-        const float x = F[n * cs + d.lin[k - n * d.count]];
-        const float ade = d.ade[k] * d.cint[k];
-        if (d.clor) {
-            const float l = d.lor[k] + d.clor[k] * d.ade[k];
-            d.lor[k] = l;
-            d.ade[k] = ade + d.cext[k] * (x - l);
-        } else {
-            d.ade[k] = ade + d.cext[k] * x;
-        }
         return;
     }
     case kLorApply: {              // k = component * cells + cell
@@ -2854,7 +2884,44 @@ __global__ __launch_bounds__(kBlock) void k_hooks(float* __restrict__ V, float* 
         s.rec[(size_t)k * 2 * s.p + ts % (2 * s.p)] = F[s.lin[k]];
         return;
     }
+    default: hook_pre(J, k, F, cs, ts);
     }
+}
+
+// ---------------------------------------------------------------------------
+// The current half step with, in workgroups of their own, the next step's
+// hooks before its voltage update: those read voltages, which the current
+// update does not set, and values that only voltage hooks use, so they need no
+// launch of their own: with it 13.7 us per step at 27 x 11 x 33, 23.0 at 72^3
+// and 29.4 at 96 x 90 x 70, without it 11.7, 20.3 and 26.9.  The field accesses
+// are the plain ones.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ void curr_hooks(const HookLaunch& L, unsigned bid, const float* __restrict__ V,
+                                           const unsigned long long cs, const unsigned* __restrict__ numts)
+{
+    unsigned k;
+    const HookJob& J = hook_job(L, bid, k);
+    if (k < J.n) hook_pre(J, k, V, cs, numts[1]);
+}
+
+template <int PM, bool CC>
+__global__ __launch_bounds__(kBlock) void k_curr_pre(const GridDesc g, float* I, const float* __restrict__ V,
+                                                     const CoefArgs k, const PmlArgs pml, unsigned* __restrict__ numts,
+                                                     const unsigned nblk, const HookLaunch L)
+{
+    if (blockIdx.x >= nblk) return curr_hooks(L, blockIdx.x - nblk, V, g.cs, numts);
+    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(numts, 1u);
+    curr_tile<PM, CC, false>(g, xcd_tile(blockIdx.x, nblk), I, V, k, pml);
+}
+
+template <int PM, bool CC, bool LT>
+__global__ __launch_bounds__(kBlock) void k_curr4_pre(const GridDesc g, const QBoxes boxes, float* I,
+                                                      const float* __restrict__ V, const CoefArgs kg, const PmlArgs pml,
+                                                      unsigned* __restrict__ numts, const unsigned nblk,
+                                                      const HookLaunch L)
+{
+    if (blockIdx.x >= nblk) return curr_hooks(L, blockIdx.x - nblk, V, g.cs, numts);
+    curr4_tile<PM, CC, false, LT>(g, boxes, blockIdx.x, nblk, I, V, kg, pml, numts);
 }
 
 // ---------------------------------------------------------------------------
@@ -3654,7 +3721,7 @@ struct ems_engine {
     float* ctab[2] = {nullptr, nullptr};
     unsigned n_unique = 0;
     CoefArgs kV{}, kI{};
-    unsigned* numts_dev = nullptr;
+    unsigned* numts_dev = nullptr;        // [0] the counter, [1] see k_hooks
     unsigned numTS = 0;
     bool inited = false;
     bool async = false;
@@ -3758,6 +3825,7 @@ struct ems_engine {
     // the current update
     std::vector<HookLaunch> hooks_pre, hooks_v, hooks_i;
     int hooks_ss = -1;
+    bool pre_ahead = false;               // k_curr_pre can take hooks_pre of the next step
 
     // probes
     std::vector<ProbeDev> probes;
@@ -5175,6 +5243,7 @@ bool mur_touches(const ems_engine* h, const HookPlan& m, unsigned long long e, b
 
 bool hooks_conflict(const ems_engine* h, const HookPlan& a, const HookPlan& b)
 {
+    if (a.d.curr != b.d.curr) return false;
     if (a.mur && b.mur) {
         if (a.face == b.face) return true;               // through the face's own values
         auto hit = [&](const HookPlan& r, const HookPlan& w) {      // w's apply sets what r's post reads
@@ -5316,8 +5385,9 @@ static int setup_hooks(ems_engine* h)
         return q;
     };
     std::vector<HookPlan> pre, v, c;
-    // before the voltage update: nothing here sets a field element, and the
-    // current side's ADE reads currents that no hook sets before the current update
+    // before the voltage update: nothing here sets a field element.  The
+    // current side's ADE reads currents, which nothing sets before the current
+    // update, and goes with the hooks after the voltage update
     for (int k = 0; k < nmur; ++k)
         if (!folded(k)) pre.push_back(mur_job(kMurPre, k));
     for (int side = 0; side < 2; ++side)
@@ -5328,7 +5398,7 @@ static int setup_hooks(ems_engine* h)
             q.d.curr = side;
             q.d.n = 3 * h->lor[k].count;
             q.d.lor = h->lor[k];
-            pre.push_back(q);
+            (side ? v : pre).push_back(q);
         }
     for (const auto& r : h->rlc) {
         HookPlan q;
@@ -5338,6 +5408,10 @@ static int setup_hooks(ems_engine* h)
         pre.push_back(q);
     }
     if ((rc = build_hook_launches(h, pre, true, h->hooks_pre))) return rc;
+    // beside the current update where that is a launch of plain accesses (with
+    // non-temporal ones a step takes 100 us and more, a launch 4); every hook
+    // here has one after the voltage update, which leaves it the timestep
+    h->pre_ahead = !h->fused && !h->nt_fields && h->hooks_pre.size() == 1;
     if (h->fused) {
         // around the quad sweep: posts, applies (the rims of the faces inside
         // the sweep), then the deferred sources; nothing else has a form there
@@ -5426,7 +5500,7 @@ static int setup_hooks(ems_engine* h)
     if (joint)
         for (auto& q : apply) q.d.kind = kMurPostApply;
     else
-        v = post;
+        v.insert(v.end(), post.begin(), post.end());
     int ss = -1;
     if (h->has_ss) {
         HookPlan q;
@@ -5729,9 +5803,12 @@ void launch_volt_t(ems_engine* h, unsigned nblk)
 }
 
 template <int PM, bool CC>
-void launch_curr_t(ems_engine* h, unsigned nblk)
+void launch_curr_t(ems_engine* h, unsigned nblk, bool pre)
 {
-    if (h->nt_fields)
+    if (pre)
+        hipLaunchKernelGGL((k_curr_pre<PM, CC>), dim3(nblk + h->hooks_pre[0].nblk), dim3(kBlock), 0, h->stream, h->g,
+                           h->I, h->V, h->kI, h->pmlI, h->numts_dev, nblk, h->hooks_pre[0]);
+    else if (h->nt_fields)
         hipLaunchKernelGGL((k_curr<PM, CC, true>), dim3(nblk), dim3(kBlock), 0, h->stream, h->g, h->I, h->V, h->kI,
                            h->pmlI, h->numts_dev);
     else
@@ -5740,21 +5817,25 @@ void launch_curr_t(ems_engine* h, unsigned nblk)
 }
 
 template <bool CC>
-void launch_update(ems_engine* h, bool curr, unsigned nblk)
+void launch_update(ems_engine* h, bool curr, unsigned nblk, bool pre)
 {
     const int pm = h->pmlV.n ? h->pml_mode : kNoPml;
-    if (pm == kPmlCompressed) curr ? launch_curr_t<kPmlCompressed, CC>(h, nblk) : launch_volt_t<kPmlCompressed, CC>(h, nblk);
-    else if (pm == kPmlPlain) curr ? launch_curr_t<kPmlPlain, CC>(h, nblk) : launch_volt_t<kPmlPlain, CC>(h, nblk);
-    else curr ? launch_curr_t<kNoPml, CC>(h, nblk) : launch_volt_t<kNoPml, CC>(h, nblk);
+    if (pm == kPmlCompressed)
+        curr ? launch_curr_t<kPmlCompressed, CC>(h, nblk, pre) : launch_volt_t<kPmlCompressed, CC>(h, nblk);
+    else if (pm == kPmlPlain) curr ? launch_curr_t<kPmlPlain, CC>(h, nblk, pre) : launch_volt_t<kPmlPlain, CC>(h, nblk);
+    else curr ? launch_curr_t<kNoPml, CC>(h, nblk, pre) : launch_volt_t<kNoPml, CC>(h, nblk);
 }
 
 template <int PM, bool CC, bool LT>
-void launch_quad_box(ems_engine* h, bool curr, const QBoxes& B, unsigned nblk, unsigned* numts)
+void launch_quad_box(ems_engine* h, bool curr, const QBoxes& B, unsigned nblk, unsigned* numts, bool pre)
 {
     if (!nblk) return;
     const size_t lds = LT ? (size_t)h->kV.ntab * sizeof(float4) : 0;
     if (curr) {
-        if (h->nt_fields)
+        if (pre)
+            hipLaunchKernelGGL((k_curr4_pre<PM, CC, LT>), dim3(nblk + h->hooks_pre[0].nblk), dim3(kBlock), lds, h->stream,
+                               h->gq, B, h->I, h->V, h->kI, h->pmlI, numts, nblk, h->hooks_pre[0]);
+        else if (h->nt_fields)
             hipLaunchKernelGGL((k_curr4<PM, CC, true, LT>), dim3(nblk), dim3(kBlock), lds, h->stream, h->gq, B, h->I,
                                h->V, h->kI, h->pmlI, numts);
         else
@@ -5771,43 +5852,44 @@ void launch_quad_box(ems_engine* h, bool curr, const QBoxes& B, unsigned nblk, u
 }
 
 template <int PM, bool CC, bool LT>
-void launch_quad_lt(ems_engine* h, bool curr)
+void launch_quad_lt(ems_engine* h, bool curr, bool pre)
 {
     if (PM != kNoPml && h->qsplit) {
         // the box without UPML cells runs without UPML code; the boxes around
-        // it (and the timestep counter) take the UPML path
-        launch_quad_box<kNoPml, CC, LT>(h, curr, h->qbox_in, h->qblk_in, nullptr);
-        launch_quad_box<PM, CC, LT>(h, curr, h->qbox_out, h->qblk_out, h->numts_dev);
+        // it (with the timestep counter and the hooks) take the UPML path
+        launch_quad_box<kNoPml, CC, LT>(h, curr, h->qbox_in, h->qblk_in, nullptr, false);
+        launch_quad_box<PM, CC, LT>(h, curr, h->qbox_out, h->qblk_out, h->numts_dev, pre);
         return;
     }
-    launch_quad_box<PM, CC, LT>(h, curr, h->qbox_all, h->qblk_all, h->numts_dev);
+    launch_quad_box<PM, CC, LT>(h, curr, h->qbox_all, h->qblk_all, h->numts_dev, pre);
 }
 
 template <int PM, bool CC>
-void launch_quad_t(ems_engine* h, bool curr)
+void launch_quad_t(ems_engine* h, bool curr, bool pre)
 {
-    if (CC && h->lds_tab) launch_quad_lt<PM, CC, true>(h, curr);
-    else launch_quad_lt<PM, CC, false>(h, curr);
+    if (CC && h->lds_tab) launch_quad_lt<PM, CC, true>(h, curr, pre);
+    else launch_quad_lt<PM, CC, false>(h, curr, pre);
 }
 
 template <bool CC>
-void launch_quad(ems_engine* h, bool curr)
+void launch_quad(ems_engine* h, bool curr, bool pre)
 {
     const int pm = h->pmlV.n ? h->pml_mode : kNoPml;
-    if (pm == kPmlCompressed) launch_quad_t<kPmlCompressed, CC>(h, curr);
-    else if (pm == kPmlPlain) launch_quad_t<kPmlPlain, CC>(h, curr);
-    else launch_quad_t<kNoPml, CC>(h, curr);
+    if (pm == kPmlCompressed) launch_quad_t<kPmlCompressed, CC>(h, curr, pre);
+    else if (pm == kPmlPlain) launch_quad_t<kPmlPlain, CC>(h, curr, pre);
+    else launch_quad_t<kNoPml, CC>(h, curr, pre);
 }
 
-void dispatch_update(ems_engine* h, bool curr, unsigned nblk)
+// pre: the current update takes the next step's pre hooks along
+void dispatch_update(ems_engine* h, bool curr, unsigned nblk, bool pre)
 {
     if (h->quad) {
-        if (h->cmp) launch_quad<true>(h, curr);
-        else launch_quad<false>(h, curr);
+        if (h->cmp) launch_quad<true>(h, curr, pre);
+        else launch_quad<false>(h, curr, pre);
         return;
     }
-    if (h->cmp) launch_update<true>(h, curr, nblk);
-    else launch_update<false>(h, curr, nblk);
+    if (h->cmp) launch_update<true>(h, curr, nblk, pre);
+    else launch_update<false>(h, curr, nblk, pre);
 }
 
 template <int PM, bool CC>
@@ -6012,8 +6094,10 @@ void lds_step(ems_engine* h)
 extern "C" {
 
 // one timestep in the reference's hook order (Engine::IterateTS, FDTD/engine.cpp:267-286,
-// priorities: UPML > default (lumped RLC, Lorentz, Mur) > excitation)
-static int launch_step(ems_engine* h, hipEvent_t* ev)
+// priorities: UPML > default (lumped RLC, Lorentz, Mur) > excitation); more:
+// another one follows before anything else may set a field; ahead: in, the
+// step before took this step's pre hooks along; out, this one took the next's
+static int launch_step(ems_engine* h, hipEvent_t* ev, bool more, bool& ahead)
 {
     if (h->fused) {
         fused_step(h, ev);
@@ -6022,13 +6106,14 @@ static int launch_step(ems_engine* h, hipEvent_t* ev)
     }
     const GridDesc& g = h->g;
     const unsigned nblk = g.qtiles * g.nzc;
-    // -- pre hooks: Mur, lumped RLC, Lorentz of both sides; UPML pre is fused
-    launch_hooks(h, h->hooks_pre, h->V, h->I);
+    // -- pre hooks: Mur, lumped RLC, Lorentz; UPML pre is fused
+    if (!ahead) launch_hooks(h, h->hooks_pre, h->V, h->I);
+    ahead = more && h->pre_ahead && !ev;
     if (ev) (void)hipEventRecord(ev[0], h->stream);
-    dispatch_update(h, false, nblk);
+    dispatch_update(h, false, nblk, false);
     if (ev) (void)hipEventRecord(ev[1], h->stream);
-    // -- post and apply hooks: Mur post, steady-state record (priority +2e6),
-    //    lumped RLC, Lorentz, Mur apply, excitation
+    // -- post and apply hooks: Lorentz pre of the currents, Mur post, steady-state
+    //    record (priority +2e6), lumped RLC, Lorentz, Mur apply, excitation
     for (size_t k = 0; k < h->hooks_v.size(); ++k) {
         launch_hook(h, h->hooks_v[k], h->V, h->I);
         if ((int)k == h->hooks_ss && h->numTS % h->ss.p == 0 && h->numTS >= 2 * h->ss.p) {
@@ -6040,7 +6125,7 @@ static int launch_step(ems_engine* h, hipEvent_t* ev)
     }
     // -- current half step: fused UPML + update, Lorentz apply, excitation
     if (ev) (void)hipEventRecord(ev[2], h->stream);
-    dispatch_update(h, true, nblk);
+    dispatch_update(h, true, nblk, ahead);
     if (ev) (void)hipEventRecord(ev[3], h->stream);
     launch_hooks(h, h->hooks_i, h->V, h->I);
     HIPCHK(hipGetLastError());
@@ -6056,8 +6141,8 @@ static void swap_pair_buffers(ems_engine* h)
 
 // the next one or two of at most `left` timesteps, and their samples: two in
 // one launch where nothing samples the state between them; ev: the events of
-// the step's (or, for a pair, its first step's) kernels
-static int advance(ems_engine* h, unsigned left, hipEvent_t* ev, unsigned* done)
+// the step's (or, for a pair, its first step's) kernels; ahead: see launch_step
+static int advance(ems_engine* h, unsigned left, hipEvent_t* ev, unsigned* done, bool& ahead)
 {
     int rc;
     bool two = h->pair && left >= 2 && !probe_due(h, h->numTS + 1);
@@ -6076,7 +6161,7 @@ static int advance(ems_engine* h, unsigned left, hipEvent_t* ev, unsigned* done)
         if (ev) (void)hipEventRecord(ev[1], h->stream);
         swap_pair_buffers(h);
         ++h->pair_launches;
-    } else if ((rc = launch_step(h, ev))) return rc;
+    } else if ((rc = launch_step(h, ev, left > 1, ahead))) return rc;
     h->numTS += *done;
     return launch_samples(h);
 }
@@ -6157,8 +6242,9 @@ static int graph_chunk(ems_engine* h, unsigned steps)
     }
     if (h->graphs.size() >= kMaxGraphs) {
         // too many distinct patterns: direct launches
+        bool ahead = false;
         for (unsigned k = 0, n; k < steps; k += n) {
-            int rc = advance(h, steps - k, nullptr, &n);
+            int rc = advance(h, steps - k, nullptr, &n, ahead);
             if (rc) return rc;
         }
         return 0;
@@ -6168,7 +6254,8 @@ static int graph_chunk(ems_engine* h, unsigned steps)
     HIPCHK(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
     int lrc = 0;
     const unsigned pairs0 = h->pair_launches;
-    for (unsigned k = 0, n; k < steps && !lrc; k += n) lrc = advance(h, steps - k, nullptr, &n);
+    bool ahead = false;
+    for (unsigned k = 0, n; k < steps && !lrc; k += n) lrc = advance(h, steps - k, nullptr, &n, ahead);
     e.pairs = h->pair_launches - pairs0;
     const hipError_t ec = hipStreamEndCapture(h->stream, &e.graph);
     if (lrc) {
@@ -6234,10 +6321,11 @@ int ems_iterate(ems_engine* h, unsigned nsteps)
     }
     HIPCHK(hipEventRecord(h->ev0, h->stream));
     unsigned s = 0;
+    bool ahead = false;                   // false after each loop: its last step takes nothing along
     // step of the events' first four, and whether that launch held two steps
     std::vector<unsigned char> pairs(nprof, 0);
     for (unsigned n; s < nprof; s += n) {
-        if ((rc = advance(h, nprof - s, &h->kev[4 * (size_t)s], &n))) return rc;
+        if ((rc = advance(h, nprof - s, &h->kev[4 * (size_t)s], &n, ahead))) return rc;
         pairs[s] = n == 2;
     }
     if (h->graph_chunk) {
@@ -6253,7 +6341,7 @@ int ems_iterate(ems_engine* h, unsigned nsteps)
         }
     }
     for (unsigned n; s < nsteps; s += n)
-        if ((rc = advance(h, nsteps - s, nullptr, &n))) return rc;
+        if ((rc = advance(h, nsteps - s, nullptr, &n, ahead))) return rc;
     HIPCHK(hipGetLastError());
     HIPCHK(hipEventRecord(h->ev1, h->stream));
     if (!h->async || nprof) {
@@ -7489,7 +7577,8 @@ int ems_adj_forward(ems_adjoint* a, unsigned nsteps, double* J)
         if (!a->kept && (rc = adj_save(a, a->ck[s]))) return rc;
         const unsigned len = std::min(a->K, nsteps - s * a->K);
         for (unsigned j = 0; j < len; ++j) {
-            rc = launch_step(h, nullptr);
+            bool ahead = false;
+            rc = launch_step(h, nullptr, false, ahead);
             ++h->numTS;
             if (rc) return rc;
             const unsigned n = s * a->K + j + 1;
@@ -7536,7 +7625,8 @@ int ems_adj_backward(ems_adjoint* a, double* dJ_dvi, double* dJ_dvv)
             if ((rc = adj_restore(a, a->ck[s]))) return rc;
             for (unsigned j = 0; j < len; ++j) {
                 adj_sample(a, (int)j, false);
-                rc = launch_step(h, nullptr);
+                bool ahead = false;
+            rc = launch_step(h, nullptr, false, ahead);
                 ++h->numTS;
                 if (rc) return rc;
             }

@@ -69,6 +69,37 @@ def test_hooks_match_oracle(gpu, name, make, steady):
     e.close()
 
 
+@pytest.mark.parametrize("quad", [False, True])
+@pytest.mark.parametrize("graph", [0, 8])
+@pytest.mark.parametrize("make", [lambda: _layers([2] * 6), lambda: _dispersive([3] * 6), lambda: _dispersive([2, 2, 0, 0, 0, 0]),
+                                  lambda: dict(scenes.mur_layers(32, 26, 22, 120), bc=[2, 3, 3, 3, 3, 3])])
+def test_calls_of_any_length_agree(gpu, make, graph, quad):
+    """The next step's hooks run beside the current update only within a call:
+    calls of one step (which never do that), calls of every length, replayed
+    chunks, and fields set between calls give the same bits."""
+    scene = make()
+    print("case hooks calls", scene["bc"], graph, quad, flush=True)
+    op = Operator(scene)
+    got = []
+    for lengths in ([1] * 45, [1, 2, 37, 3, 2], [40, 5]):
+        # quad: the four-cell kernels where the rows allow them, else the engine's choice
+        eng = EngineHIP(op, fused=False, quad=quad if scene["lines"][0].size % 4 == 0 else None)
+        eng.set_graph(graph)
+        n = 0
+        for k in lengths:
+            if n == 40:                # a field set between two calls
+                v = eng.get_volt()
+                eng.set_volt(np.ascontiguousarray(v * np.float32(0.5)))
+            eng.IterateTS(k)
+            n += k
+        got.append((eng.get_volt(), eng.get_curr()))
+        eng.close()
+    assert np.max(np.abs(got[0][0])) > 0
+    for v, c in got[1:]:
+        assert np.array_equal(v, got[0][0])
+        assert np.array_equal(c, got[0][1])
+
+
 @pytest.mark.parametrize("nprobe", [1, 191, 400])
 def test_steady_state_of_many_probes(gpu, nprobe):
     """More probes than the evaluation has threads, and one."""
