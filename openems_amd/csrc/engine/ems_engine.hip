@@ -2567,8 +2567,8 @@ struct MurDev {
 // The current update (curr_tile's arithmetic, FDTD/engine.cpp:170-222) redone
 // from the final voltages V1 and the currents of state n, into I1, for the
 // quad sweep's currents that read voltages set after the sweep: the planes
-// lo..hi along `axis` next to a Mur face (k_curr_band), and the cells next to
-// a deferred voltage source (k_curr_cells).
+// lo..hi along `axis` next to a Mur face, and the cells next to
+// a deferred voltage source (k_curr_again).
 __device__ __forceinline__ void curr_cell(const GridDesc& g, const float* __restrict__ V1, const float* __restrict__ I0,
                                           float* __restrict__ I1, const CoefArgs& k, unsigned long long p)
 {
@@ -2601,33 +2601,6 @@ __device__ __forceinline__ void curr_cell(const GridDesc& g, const float* __rest
         f = f + b[m] * curl[m];
         I1[m * cs + p] = f;
     }
-}
-
-// the same at listed cells (each with x, y, z below the last line)
-__global__ void k_curr_cells(const GridDesc g, const float* __restrict__ V1, const float* __restrict__ I0,
-                             float* __restrict__ I1, const CoefArgs k, const unsigned long long* __restrict__ cells,
-                             unsigned n)
-{
-    const unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) curr_cell(g, V1, I0, I1, k, cells[t]);
-}
-
-__global__ void k_curr_band(const GridDesc g, const float* __restrict__ V1, const float* __restrict__ I0,
-                            float* __restrict__ I1, const CoefArgs k, int axis, unsigned lo, unsigned hi)
-{
-    const unsigned n[3] = {axis == 0 ? hi - lo + 1 : g.Nx, axis == 1 ? hi - lo + 1 : g.Ny,
-                           axis == 2 ? hi - lo + 1 : g.Nz};
-    const unsigned long long cnt = (unsigned long long)n[0] * n[1] * n[2];
-    const unsigned long long t = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= cnt) return;
-    unsigned c[3];
-    c[0] = (unsigned)(t % n[0]);
-    c[1] = (unsigned)((t / n[0]) % n[1]);
-    c[2] = (unsigned)(t / ((unsigned long long)n[0] * n[1]));
-    c[axis] += lo;
-    const unsigned x = c[0], y = c[1], z = c[2];
-    if (x + 1 >= g.Nx || y + 1 >= g.Ny || z + 1 >= g.Nz) return;
-    curr_cell(g, V1, I0, I1, k, x + (unsigned long long)g.Nx * y + (unsigned long long)g.plane * z);
 }
 
 // ---------------------------------------------------------------------------
@@ -2889,13 +2862,30 @@ __global__ __launch_bounds__(kBlock) void k_hooks(float* __restrict__ V, float* 
 }
 
 // ---------------------------------------------------------------------------
-// The current half step with, in workgroups of their own, the next step's
-// hooks before its voltage update: those read voltages, which the current
-// update does not set, and values that only voltage hooks use, so they need no
-// launch of their own: with it 13.7 us per step at 27 x 11 x 33, 23.0 at 72^3
-// and 29.4 at 96 x 90 x 70, without it 11.7, 20.3 and 26.9.  The field accesses
-// are the plain ones.
+// After the hooks of a single-sweep step: the currents of up to six bands of
+// planes next to faces and of listed cells again, each a job of workgroups, in
+// one launch with the next step's hooks before its voltage update (whose
+// voltages are final) and, where no hook follows, the timestep's advance.  The
+// sweep writes out of place, so where bands meet the same value is stored
+// twice.  Each job is a few microseconds beside the sweep's 880: 512 x 384 x
+// 320 layers TIMES.
 // ---------------------------------------------------------------------------
+constexpr unsigned kMaxBands = 6;  // of one launch
+
+struct CurrBand {
+    int axis;
+    unsigned lo, hi;               // first and last plane
+    unsigned first;                // first workgroup
+};
+
+struct CurrAgain {
+    CurrBand band[kMaxBands];
+    unsigned nband;
+    const unsigned long long* cells;   // each with x, y, z below the last line
+    unsigned ncells, first;            // of the listed cells
+    unsigned nblk;                     // workgroups before the hooks'
+};
+
 __device__ __forceinline__ void curr_hooks(const HookLaunch& L, unsigned bid, const float* __restrict__ V,
                                            const unsigned long long cs, const unsigned* __restrict__ numts)
 {
@@ -2904,6 +2894,42 @@ __device__ __forceinline__ void curr_hooks(const HookLaunch& L, unsigned bid, co
     if (k < J.n) hook_pre(J, k, V, cs, numts[1]);
 }
 
+__global__ __launch_bounds__(kBlock) void k_curr_again(const GridDesc g, const float* __restrict__ V1,
+                                                       const float* __restrict__ I0, float* __restrict__ I1,
+                                                       const CoefArgs k, const CurrAgain A, const HookLaunch L,
+                                                       unsigned* __restrict__ numts, int tick)
+{
+    const unsigned bid = blockIdx.x;
+    if (bid >= A.nblk) return curr_hooks(L, bid - A.nblk, V1, g.cs, numts);
+    if (tick && bid == 0 && threadIdx.x == 0) numts[0] = numts[0] + 1u;
+    if (bid >= A.first) {
+        const unsigned t = (bid - A.first) * kBlock + threadIdx.x;
+        if (t < A.ncells) curr_cell(g, V1, I0, I1, k, A.cells[t]);
+        return;
+    }
+    CurrBand b = A.band[0];
+#pragma unroll
+    for (unsigned j = 1; j < kMaxBands; ++j)
+        if (j < A.nband && bid >= A.band[j].first) b = A.band[j];
+    const unsigned d = b.hi - b.lo + 1;
+    const unsigned n0 = b.axis == 0 ? d : g.Nx, n1 = b.axis == 1 ? d : g.Ny, n2 = b.axis == 2 ? d : g.Nz;
+    const unsigned t = (bid - b.first) * kBlock + threadIdx.x;
+    const unsigned r = t / n0, zr = r / n1;
+    if (zr >= n2) return;
+    const unsigned x = t - r * n0 + (b.axis == 0 ? b.lo : 0u), y = r - zr * n1 + (b.axis == 1 ? b.lo : 0u);
+    const unsigned z = zr + (b.axis == 2 ? b.lo : 0u);
+    if (x + 1 >= g.Nx || y + 1 >= g.Ny || z + 1 >= g.Nz) return;
+    curr_cell(g, V1, I0, I1, k, x + (unsigned long long)g.Nx * y + (unsigned long long)g.plane * z);
+}
+
+// ---------------------------------------------------------------------------
+// The current half step with, in workgroups of their own, the next step's
+// hooks before its voltage update: those read voltages, which the current
+// update does not set, and values that only voltage hooks use, so they need no
+// launch of their own: with it 13.7 us per step at 27 x 11 x 33, 23.0 at 72^3
+// and 29.4 at 96 x 90 x 70, without it 11.7, 20.3 and 26.9.  The field accesses
+// are the plain ones.
+// ---------------------------------------------------------------------------
 template <int PM, bool CC>
 __global__ __launch_bounds__(kBlock) void k_curr_pre(const GridDesc g, float* I, const float* __restrict__ V,
                                                      const CoefArgs k, const PmlArgs pml, unsigned* __restrict__ numts,
@@ -3812,6 +3838,7 @@ struct ems_engine {
     // changes it after the sweep, outside the bands (linear cell indices)
     unsigned long long* cell_list = nullptr;
     unsigned ncells = 0;
+    std::vector<CurrAgain> curr_again;    // both, as the jobs of launches
     // lumped RLC and dispersive lists
     std::vector<RlcDev> rlc;
     std::vector<LorDev> lor;
@@ -5412,6 +5439,26 @@ static int setup_hooks(ems_engine* h)
     // non-temporal ones a step takes 100 us and more, a launch 4); every hook
     // here has one after the voltage update, which leaves it the timestep
     h->pre_ahead = !h->fused && !h->nt_fields && h->hooks_pre.size() == 1;
+    if (h->fused && nmur) {
+        h->curr_again.clear();
+        for (size_t k = 0; k < h->bands.size() || (h->ncells && k == h->bands.size()); ++k) {
+            if (h->curr_again.empty() || (k < h->bands.size() && k % kMaxBands == 0)) h->curr_again.push_back(CurrAgain{});
+            CurrAgain& A = h->curr_again.back();
+            unsigned long long cnt = h->ncells;
+            if (k < h->bands.size()) {
+                const auto& b = h->bands[k];
+                A.band[A.nband++] = CurrBand{b.axis, b.lo, b.hi, A.nblk};
+                cnt = (unsigned long long)(b.hi - b.lo + 1) * h->N[0] * h->N[1] * h->N[2] / h->N[b.axis];
+                A.first = A.nblk + (unsigned)((cnt + kBlock - 1) / kBlock);
+            } else {
+                A.cells = h->cell_list;
+                A.ncells = h->ncells;
+            }
+            A.nblk += (unsigned)((cnt + kBlock - 1) / kBlock);
+        }
+        // beside the currents done again
+        h->pre_ahead = !h->curr_again.empty() && h->hooks_pre.size() == 1;
+    }
     if (h->fused) {
         // around the quad sweep: posts, applies (the rims of the faces inside
         // the sweep), then the deferred sources; nothing else has a form there
@@ -6021,11 +6068,12 @@ void launch_hooks(ems_engine* h, const std::vector<HookLaunch>& hooks, float* V,
 
 // one fused step from state n (h->V, h->I, current fluxes) into the second
 // buffers, which then become the current state
-void fused_step(ems_engine* h, hipEvent_t* ev)
+void fused_step(ems_engine* h, hipEvent_t* ev, bool more, bool& ahead)
 {
-    const unsigned T = 256;
     // Mur pre hooks read state n (FDTD/engine.cpp:224-265 order; only the quad sweep has Mur)
-    launch_hooks(h, h->hooks_pre, h->V, h->I);
+    if (!ahead) launch_hooks(h, h->hooks_pre, h->V, h->I);
+    ahead = more && h->pre_ahead && !ev;
+    bool tick = true;
     if (ev) (void)hipEventRecord(ev[0], h->stream);
     if (h->fused == 3) quad_step(h);
     else if (h->fused == 2) column_step(h);
@@ -6039,18 +6087,17 @@ void fused_step(ems_engine* h, hipEvent_t* ev)
         // Mur apply, the deferred voltage sources, then the current update of
         // the planes next to each face again, with their current sources
         launch_hooks(h, h->hooks_v, h->V_alt, h->I_alt);
-        for (const auto& b : h->bands) {
-            const unsigned long long cnt = (unsigned long long)(b.hi - b.lo + 1) * h->N[0] * h->N[1] * h->N[2] /
-                                           h->N[b.axis];
-            hipLaunchKernelGGL(k_curr_band, dim3((unsigned)((cnt + T - 1) / T)), dim3(T), 0, h->stream, h->g,
-                               h->V_alt, h->I, h->I_alt, h->kI, b.axis, b.lo, b.hi);
+        for (size_t k = 0; k < h->curr_again.size(); ++k) {
+            const CurrAgain& A = h->curr_again[k];
+            const bool last = k + 1 == h->curr_again.size();
+            const HookLaunch L = last && ahead ? h->hooks_pre[0] : HookLaunch{};
+            if (last) tick = !h->hooks_i.empty();
+            hipLaunchKernelGGL(k_curr_again, dim3(A.nblk + L.nblk), dim3(kBlock), 0, h->stream, h->g, h->V_alt, h->I,
+                               h->I_alt, h->kI, A, L, h->numts_dev, last && !tick ? 1 : 0);
         }
-        if (h->ncells)
-            hipLaunchKernelGGL(k_curr_cells, dim3((h->ncells + T - 1) / T), dim3(T), 0, h->stream, h->g, h->V_alt,
-                               h->I, h->I_alt, h->kI, h->cell_list, h->ncells);
         launch_hooks(h, h->hooks_i, h->V_alt, h->I_alt);
     }
-    hipLaunchKernelGGL(k_tick, dim3(1), dim3(64), 0, h->stream, h->numts_dev);
+    if (tick) hipLaunchKernelGGL(k_tick, dim3(1), dim3(64), 0, h->stream, h->numts_dev);
     if (ev) (void)hipEventRecord(ev[3], h->stream);
     swap_step_buffers(h);
 }
@@ -6100,7 +6147,7 @@ extern "C" {
 static int launch_step(ems_engine* h, hipEvent_t* ev, bool more, bool& ahead)
 {
     if (h->fused) {
-        fused_step(h, ev);
+        fused_step(h, ev, more, ahead);
         HIPCHK(hipGetLastError());
         return 0;
     }

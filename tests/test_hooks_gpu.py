@@ -69,27 +69,37 @@ def test_hooks_match_oracle(gpu, name, make, steady):
     e.close()
 
 
-@pytest.mark.parametrize("quad", [False, True])
+def _sweep_mur(nx, faces=(2, 2, 2, 2, 2, 2)):
+    return lambda: dict(scenes.mur_layers(nx, 26, 22, 120), bc=list(faces))
+
+
 @pytest.mark.parametrize("graph", [0, 8])
-@pytest.mark.parametrize("make", [lambda: _layers([2] * 6), lambda: _dispersive([3] * 6), lambda: _dispersive([2, 2, 0, 0, 0, 0]),
-                                  lambda: dict(scenes.mur_layers(32, 26, 22, 120), bc=[2, 3, 3, 3, 3, 3])])
-def test_calls_of_any_length_agree(gpu, make, graph, quad):
-    """The next step's hooks run beside the current update only within a call:
-    calls of one step (which never do that), calls of every length, replayed
-    chunks, and fields set between calls give the same bits."""
+@pytest.mark.parametrize("make,kw", [
+    (lambda: _layers([2] * 6), dict(fused=False)),
+    (lambda: _dispersive([3] * 6), dict(fused=False, quad=False)),
+    (lambda: _dispersive([3] * 6), dict(fused=False, quad=True)),
+    (lambda: _dispersive([2, 2, 0, 0, 0, 0]), dict(fused=False)),
+    (_sweep_mur(32, (2, 3, 3, 3, 3, 3)), dict(fused=False, quad=True)),
+    (_sweep_mur(32), dict(fused="quads")),
+    (_sweep_mur(264), dict(fused="quads")),                              # the x faces inside the sweep
+    (_sweep_mur(264, (2, 2, 0, 0, 0, 0)), dict(fused="quads")),          # no face left around it
+    (_sweep_mur(264, (0, 0, 0, 0, 0, 2)), dict(fused="quads")),
+], ids=["layers", "ade_pml", "ade_pml_quads", "ade_mur", "mur_pml", "sweep", "sweep_fold", "sweep_fold_only", "sweep_z"])
+def test_calls_of_any_length_agree(gpu, make, kw, graph):
+    """The next step's hooks run beside the currents only within a call: calls
+    of one step (which never do that), calls of every length, replayed chunks,
+    and fields set between calls give the same bits."""
     scene = make()
-    print("case hooks calls", scene["bc"], graph, quad, flush=True)
+    print("case hooks calls", scene["bc"], kw, graph, flush=True)
     op = Operator(scene)
     got = []
     for lengths in ([1] * 45, [1, 2, 37, 3, 2], [40, 5]):
-        # quad: the four-cell kernels where the rows allow them, else the engine's choice
-        eng = EngineHIP(op, fused=False, quad=quad if scene["lines"][0].size % 4 == 0 else None)
+        eng = EngineHIP(op, **kw)
         eng.set_graph(graph)
         n = 0
         for k in lengths:
             if n == 40:                # a field set between two calls
-                v = eng.get_volt()
-                eng.set_volt(np.ascontiguousarray(v * np.float32(0.5)))
+                eng.set_volt(np.ascontiguousarray(eng.get_volt() * np.float32(0.5)))
             eng.IterateTS(k)
             n += k
         got.append((eng.get_volt(), eng.get_curr()))
