@@ -996,7 +996,7 @@ struct StepArgs {
     CoefArgs kV, kI;
     PmlArgs pV, pI;
     ExcArgs eV, eI;
-    const unsigned* numts;         // [0] timestep counter (advanced by k_tick after the step)
+    const unsigned* numts;         // [0] timestep counter (advanced by k_tick or k_curr_again after the step)
 };
 
 template <int PM, bool CC>
@@ -1218,7 +1218,7 @@ struct Step2Args {
     CoefArgs kV, kI;
     PmlArgs pV, pI;                // one slab table and index array for both halves
     ExcArgs eV, eI;                // beg: [plane + 1] per-column ranges
-    const unsigned* numts;         // [0] timestep counter (advanced by k_tick after the step)
+    const unsigned* numts;         // [0] timestep counter (advanced by k_tick or k_curr_again after the step)
 };
 
 // main coefficients (c, v) of component n at cell p: plain arrays or table
@@ -2665,7 +2665,7 @@ struct SteadyDev {
 // detection (96 x 90 x 70) 22 -> 5 and 64.7 -> 26.9 us; Drude, Lorentz and
 // Debye boxes with RLC elements (72^3) 17 -> 4 and 38.2 -> 20.3 us; one Mur
 // face (27 x 11 x 33) 6 -> 3 and 17.3 -> 11.7 us; 512 x 384 x 320 layers
-// around the quad sweep, which has no such update, 0.984 -> 0.959 ms.
+// around the quad sweep (beside k_curr_again) 0.976 -> 0.934 ms.
 //
 //   MurPre / MurPost / MurApply  Engine_Ext_Mur_ABC (engine_ext_mur_abc.cpp:68-178);
 //                  the faces' applies run in reverse creation order, so where
@@ -2867,8 +2867,8 @@ __global__ __launch_bounds__(kBlock) void k_hooks(float* __restrict__ V, float* 
 // one launch with the next step's hooks before its voltage update (whose
 // voltages are final) and, where no hook follows, the timestep's advance.  The
 // sweep writes out of place, so where bands meet the same value is stored
-// twice.  Each job is a few microseconds beside the sweep's 880: 512 x 384 x
-// 320 layers TIMES.
+// twice.  One launch each, on 512 x 384 x 320 layers, took 0.955 ms per step,
+// this 0.934, of which the sweep is 0.867 and the hooks 0.020.
 // ---------------------------------------------------------------------------
 constexpr unsigned kMaxBands = 6;  // of one launch
 
