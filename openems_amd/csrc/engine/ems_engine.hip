@@ -5249,23 +5249,35 @@ namespace {
 struct HookPlan {
     HookJob d{};
     std::vector<unsigned long long> cells;    // sorted component * cs + cell of a list job
+    std::vector<unsigned char> lines[3];      // per axis and line: bit c where component c has such an element
     bool writes = true;                       // it sets field elements
     const ems_engine::MurGeo* mur = nullptr;  // a Mur face's job
     int face = -1;
 };
 
-// element e on the lines a Mur job reads (its neighbour line, before or
-// after the update) or sets (its face line)
-bool mur_touches(const ems_engine* h, const HookPlan& m, unsigned long long e, bool want_write)
+// the lines that a list job's elements lie on
+void find_lines(const ems_engine* h, HookPlan& q)
 {
-    const int c = (int)(e / h->cs);
-    if (c == m.mur->ny) return false;
-    const unsigned long long p = e % h->cs;
-    const unsigned x[3] = {(unsigned)(p % h->N[0]), (unsigned)(p / h->N[0] % h->N[1]), (unsigned)(p / h->g.plane)};
-    const unsigned v = x[m.mur->ny];
-    const bool reads = m.d.kind != kMurApply && v == m.mur->shift;
-    const bool sets = m.d.kind != kMurPost && v == m.mur->line;
-    return want_write ? sets : reads || sets;
+    for (int n = 0; n < 3; ++n) q.lines[n].assign(h->N[n], 0);
+    for (unsigned long long e : q.cells) {
+        const unsigned c = e >= 2 * h->cs ? 2u : e >= h->cs ? 1u : 0u;
+        const unsigned p = (unsigned)(e - c * h->cs), z = p / h->g.plane, r = p - z * h->g.plane, y = r / h->N[0];
+        const unsigned char bit = (unsigned char)(1u << c);
+        q.lines[0][r - y * h->N[0]] |= bit;
+        q.lines[1][y] |= bit;
+        q.lines[2][z] |= bit;
+    }
+}
+
+// an element of list job l on the line that Mur job m reads (the neighbour
+// line, before or after the update; only if l sets it) or sets (the face line)
+bool mur_touches(const HookPlan& m, const HookPlan& l)
+{
+    const auto& on = l.lines[m.mur->ny];
+    if (on.empty()) return false;
+    const unsigned tangential = 7u & ~(1u << m.mur->ny);
+    return (m.d.kind != kMurPost && (on[m.mur->line] & tangential)) ||
+           (l.writes && m.d.kind != kMurApply && (on[m.mur->shift] & tangential));
 }
 
 bool hooks_conflict(const ems_engine* h, const HookPlan& a, const HookPlan& b)
@@ -5285,9 +5297,7 @@ bool hooks_conflict(const ems_engine* h, const HookPlan& a, const HookPlan& b)
     if (a.mur || b.mur) {
         const HookPlan& m = a.mur ? a : b;
         const HookPlan& l = a.mur ? b : a;
-        for (unsigned long long e : l.cells)
-            if (mur_touches(h, m, e, !l.writes)) return true;
-        return false;
+        return mur_touches(m, l);
     }
     if (!a.writes && !b.writes) return false;
     for (size_t i = 0, j = 0; i < a.cells.size() && j < b.cells.size();) {
@@ -5370,6 +5380,7 @@ static long mur_over(const ems_engine* h, int k, int c, std::vector<unsigned cha
 
 static int setup_hooks(ems_engine* h)
 {
+    const int nmur = (int)h->mur.size();
     auto mur_job = [&](int kind, int k) {
         HookPlan q;
         q.d.kind = kind;
@@ -5394,9 +5405,9 @@ static int setup_hooks(ems_engine* h)
         q.d.ts_bias = bias;
         q.cells = e.h_glin;
         std::sort(q.cells.begin(), q.cells.end());
+        if (!curr && nmur) find_lines(h, q);
         return q;
     };
-    const int nmur = (int)h->mur.size();
     auto folded = [&](int k) { return k == h->mur_fold[0] || k == h->mur_fold[1]; };
     int rc;
     std::vector<unsigned char> over;
@@ -5490,6 +5501,7 @@ static int setup_hooks(ems_engine* h)
         q.d.rlc = h->rlc[k];
         q.cells = h->h_rlc[k];
         std::sort(q.cells.begin(), q.cells.end());
+        if (nmur) find_lines(h, q);
         list.push_back(q);
     }
     auto lor_apply = [&](int side, HookPlan& q) {
@@ -5517,6 +5529,7 @@ static int setup_hooks(ems_engine* h)
         if (!q.d.n) return 0;
         for (int n = 0; n < 3; ++n)
             for (unsigned x : cell) q.cells.push_back(n * h->cs + x);
+        if (!side && nmur) find_lines(h, q);
         unsigned *dc, *db;
         LorTerm* dt;
         int r;
@@ -5557,6 +5570,7 @@ static int setup_hooks(ems_engine* h)
         q.writes = false;
         q.cells = h->h_ss;
         std::sort(q.cells.begin(), q.cells.end());
+        if (nmur) find_lines(h, q);
         ss = (int)v.size();
         v.push_back(q);
     }
