@@ -366,7 +366,9 @@ void ems_destroy(ems_engine* h);
  * the same timestep, and carry no Mur, Lorentz, lumped RLC or field dump.  The
  * batch does not own them: destroy it before them.  While batched, advance the
  * engines only through ems_batch_iterate; ems_probe_results / ems_get_volt /
- * ems_get_curr on each engine read its results. */
+ * ems_get_curr on each engine read its results.  Engines that advance two
+ * timesteps per launch (ems_get_pair) take single steps from here on, and give
+ * back the buffers that pairs need. */
 typedef struct ems_batch ems_batch;
 int ems_batch_create(ems_batch** out, ems_engine* const* engines, unsigned count);
 /* tile_x: 0 = 256 consecutive plane positions per workgroup, else tile_x x

@@ -6200,6 +6200,27 @@ static void swap_pair_buffers(ems_engine* h)
     std::swap(h->numts_dev, h->numts_alt);
 }
 
+// The engine advances by single steps from now on, on the buffers that hold
+// its state now; the ones that only pairs need are freed.
+static void leave_pairs(ems_engine* h)
+{
+    if (!h->pair) return;
+    (void)hipStreamSynchronize(h->stream);
+    drop_graphs(h);
+    h->pair = false;
+    auto release = [&](float*& p) {
+        if (!p) return;
+        h->allocs.erase(std::find(h->allocs.begin(), h->allocs.end(), (void*)p));
+        (void)hipFree(p);
+        p = nullptr;
+    };
+    if (!h->fused) {             // the quad sweep's second fields stay
+        release(h->V_alt);
+        release(h->I_alt);
+    }
+    for (float*& f : h->flux_alt) release(f);
+}
+
 // the next one or two of at most `left` timesteps, and their samples: two in
 // one launch where nothing samples the state between them; ev: the events of
 // the step's (or, for a pair, its first step's) kernels; ahead: see launch_step
@@ -6965,6 +6986,9 @@ int ems_batch_create(ems_batch** out, ems_engine* const* engines, unsigned count
             if (engines[j] == e) return fail(EMS_E_ARG, "an engine appears twice in the batch");
     }
     HIPCHK(hipSetDevice(e0->device));
+    // an instance names its engine's field, flux and counter buffers for good:
+    // an engine that went on advancing in pairs by itself would swap them
+    for (unsigned i = 0; i < count; ++i) leave_pairs(engines[i]);
     ems_batch* b = new ems_batch();
     auto bail = [&](int r) {
         ems_batch_destroy(b);

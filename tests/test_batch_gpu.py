@@ -2,10 +2,13 @@
 instance of a batch of uneven grids is bit-identical to the oracle engine
 and to its own engine run alone, for the autotuned and for hand-set tile
 shapes, z depths and grid sizes."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 from openems_amd import scenes
+from openems_amd._native import check, lib
 from openems_amd.batch import BatchEngine
 from openems_amd.simulation import Simulation
 from oracle.operator_ref import RefOperator
@@ -93,6 +96,42 @@ def test_batch_equals_engines_alone(gpu, config):
     b.iterate(50)
     _check_same(b, ref, 90)
     b.close()
+
+
+@pytest.mark.parametrize("pml", [True, False])
+def test_batch_of_engines_that_advanced_in_pairs(gpu, monkeypatch, pml):
+    """Automatic engines, one pair of timesteps each (their state and counter
+    in the second buffers), batched; then steps of the batch and of the
+    engines by themselves in turn."""
+    monkeypatch.setenv("EMS_PAIR", "1")
+    scs = _small_batch(3, 60, seed=5)
+    if not pml:
+        for s in scs:
+            s["bc"] = [0] * 6
+    print("case batch after pairs, UPML", pml, flush=True)
+    ref = [_alone(s, 21) for s in scs]
+    sims = [Simulation(s, layout="compressed") for s in scs]
+    for sim in sims:
+        sim.eng.IterateTS(2)
+        assert sim.eng.pair()[0] == 1 and sim.eng.pair()[2] == 1
+    hs = (C.c_void_p * len(sims))(*[sim.eng.h.value for sim in sims])
+    b = C.c_void_p()
+    check(lib().ems_batch_create(C.byref(b), hs, len(sims)))
+    check(lib().ems_batch_iterate(b, 5))
+    for sim in sims:
+        sim.eng.IterateTS(6)
+    check(lib().ems_batch_iterate(b, 8))
+    for sim, (v, c, probes) in zip(sims, ref):
+        assert sim.eng.numTS == 21
+        assert np.max(np.abs(v)) > 0
+        assert np.array_equal(sim.eng.get_volt(), v) and np.array_equal(sim.eng.get_curr(), c)
+        got = sim.results()["probes"]
+        for name, p in probes.items():
+            assert np.array_equal(got[name]["td"], p["td"])
+        assert sim.eng.pair()[0] == 0
+    lib().ems_batch_destroy(b)
+    for sim in sims:
+        sim.close()
 
 
 def test_batch_refuses_mixed_layouts(gpu):
