@@ -5185,6 +5185,11 @@ static int setup_pair(ems_engine* h)
     // sources: lists per column ordered by plane, their planes, and the tiles
     // (rims included) that hold one
     std::vector<unsigned> mask((a.ntiles + 31) / 32, 0u);
+    const unsigned nty = a.ntiles / a.ntx;
+    // first and last of the n tiles of t lines that hold line x
+    auto tiles_of = [](unsigned x, unsigned t, unsigned n) {
+        return std::make_pair(x < t ? 0u : (x - t) / (t - 3u) + 1u, std::min(x / (t - 3u), n - 1u));
+    };
     bool any = false;
     for (int c = 0; c < 2; ++c) {
         const auto& host = h->exc[c].host;
@@ -5192,23 +5197,28 @@ static int setup_pair(ems_engine* h)
         a.sz[c][1] = 0;
         if (host.empty()) continue;
         any = true;
-        std::vector<ExcEnt> ent(host);
-        std::stable_sort(ent.begin(), ent.end(), [&](const ExcEnt& l, const ExcEnt& r) {
-            const unsigned cl = l.x + N[0] * (unsigned)l.y, cr = r.x + N[0] * (unsigned)r.y;
-            return cl != cr ? cl < cr : l.z < r.z;
-        });
         std::vector<unsigned> beg(h->g.plane + 1, 0);
         unsigned lo = ~0u, hi = 0;
-        for (const auto& e : ent) {
+        for (const auto& e : host) {
             ++beg[e.x + N[0] * (unsigned)e.y + 1];
             lo = std::min(lo, (unsigned)e.z);
             hi = std::max(hi, (unsigned)e.z);
-            for (unsigned t = 0; t < a.ntiles; ++t) {
-                const unsigned X0 = t % a.ntx * (a.tx - 3u), Y0 = t / a.ntx * (a.ty - 3u);
-                if (e.x >= X0 && e.x < X0 + a.tx && e.y >= Y0 && e.y < Y0 + a.ty) mask[t >> 5] |= 1u << (t & 31);
-            }
+            const std::pair<unsigned, unsigned> tx = tiles_of(e.x, a.tx, a.ntx), ty = tiles_of(e.y, a.ty, nty);
+            for (unsigned j = ty.first; j <= ty.second; ++j)
+                for (unsigned i = tx.first; i <= tx.second; ++i) {
+                    const unsigned t = i + a.ntx * j;
+                    mask[t >> 5] |= 1u << (t & 31);
+                }
         }
         for (size_t i = 1; i < beg.size(); ++i) beg[i] += beg[i - 1];
+        std::vector<ExcEnt> ent(host.size());
+        std::vector<unsigned> at(beg);
+        for (const auto& e : host) ent[at[e.x + N[0] * (unsigned)e.y]++] = e;
+        auto below = [](const ExcEnt& l, const ExcEnt& r) { return l.z < r.z; };
+        for (size_t i = 0; i < h->g.plane; ++i) {
+            const auto b = ent.begin() + beg[i], e = ent.begin() + beg[i + 1];
+            if (!std::is_sorted(b, e, below)) std::stable_sort(b, e, below);
+        }
         a.sz[c][0] = lo;
         a.sz[c][1] = hi;
         unsigned* db;

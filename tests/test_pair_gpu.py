@@ -4,6 +4,8 @@ anywhere, chunks down to one plane, sources (voltage and current) on rims and
 chunk ends, UPML in both layouts with slab faces inside tiles and hook-only
 cells from random fields, both coefficient layouts, odd step counts, samples
 that force single steps between pairs, and graph replays of either parity."""
+import time
+
 import numpy as np
 import pytest
 
@@ -127,3 +129,25 @@ def test_pair_policy(gpu, monkeypatch):
         eng = EngineHIP(op, **kw)
         assert eng.pair()[0] == want, (op.N, kw)
         eng.close()
+
+
+def test_sheet_source_over_many_tiles(gpu, monkeypatch):
+    """A source in every column of 600 x 600 and 14400 tiles: set-up does not
+    test every column against every tile (12.9 s; as it is 0.08 s)."""
+    monkeypatch.setenv("EMS_PAIR", "1")
+    op = Operator(_sheet(600, 600, 4))
+    half = EngineHIP(op, fused=False)
+    half.IterateTS(7)
+    monkeypatch.setenv("EMS_PAIR_TILE", "8,8,4")
+    print("case pairs sheet source set-up", flush=True)
+    t = time.perf_counter()
+    eng = EngineHIP(op)
+    t = time.perf_counter() - t
+    print("set-up %.2f s" % t, flush=True)
+    assert eng.pair()[0] == 1
+    assert t < 3.0
+    eng.IterateTS(7)
+    assert np.max(np.abs(half.get_volt())) > 0
+    assert np.array_equal(eng.get_volt(), half.get_volt()) and np.array_equal(eng.get_curr(), half.get_curr())
+    eng.close()
+    half.close()
