@@ -3874,6 +3874,7 @@ struct ems_engine {
     double* energy_part = nullptr;
     unsigned read_rows = 0;         // x planes that read_buf holds
     float* read_buf = nullptr;      // of get_field; not in allocs, whose growth drops the captured chunks
+    std::mutex read_mu;             // the read-out that uses it
 
     // steady-state detection
     bool has_ss = false;
@@ -6490,7 +6491,8 @@ static int get_field(ems_engine* h, const float* d, float* out)
     if (!h || !out) return fail(EMS_E_ARG, "null argument");
     HIPCHK(hipSetDevice(h->device));
     HIPCHK(hipStreamSynchronize(h->stream));
-    // turned on the device, kReadBytes at a time
+    // turned on the device, kReadBytes at a time; several threads may read at once
+    std::lock_guard<std::mutex> lk(h->read_mu);
     const unsigned *N = h->N;
     const size_t row = (size_t)N[1] * N[2];              // floats of one x
     if (!h->read_buf) {

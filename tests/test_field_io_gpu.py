@@ -3,6 +3,8 @@
 Engine::GetVolt / SetVolt over a box; ems_get_field_at, the reference's
 Engine_Interface_FDTD::GetEField / GetHField with its three interpolation
 types), against the whole-field reads and the device field dumps."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -81,3 +83,33 @@ def test_field_at_matches_td_dump(gpu, field, interp):
         checked += 1
     assert checked >= 4 and np.abs(td[k]).max() > 0
     sim.close()
+
+
+def test_fields_read_by_several_threads(gpu):
+    """Threads that read one engine's fields at once, the first read-out among
+    them, each get the whole field they asked for."""
+    op = Operator(dict(scenes.pec_cavity(8, 10), lines=[np.arange(n, dtype=np.float64) for n in (90, 70, 50)], probes=[]))
+    rng = np.random.default_rng(3)
+    want = [rng.standard_normal((3,) + tuple(op.N)).astype(np.float32) for _ in range(2)]
+    bad = []
+    print("case fields read by 4 threads", flush=True)
+    for _ in range(3):
+        eng = EngineHIP(op)
+        eng.set_volt(want[0])
+        eng.set_curr(want[1])
+        start = threading.Barrier(4)
+
+        def read(k):
+            start.wait()
+            for j in range(8):
+                c = (k + j) % 2
+                if not np.array_equal((eng.get_curr if c else eng.get_volt)(), want[c]):
+                    bad.append((k, j))
+
+        th = [threading.Thread(target=read, args=(k,)) for k in range(4)]
+        for t in th:
+            t.start()
+        for t in th:
+            t.join()
+        eng.close()
+    assert not bad
