@@ -3730,6 +3730,12 @@ void parallel_rows(size_t n, const std::function<void(size_t, size_t)>& fn);
 // ---------------------------------------------------------------------------
 // engine state
 // ---------------------------------------------------------------------------
+struct ems_engine;
+
+// Device memory for engine h or what works on it.  Where there is none left,
+// the buffers that only pairs of timesteps need make room.
+static hipError_t device_malloc(ems_engine* h, void** q, size_t bytes);
+
 struct ems_engine {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -3751,7 +3757,12 @@ struct ems_engine {
     unsigned numTS = 0;
     bool inited = false;
     bool async = false;
-    std::vector<void*> allocs;
+    struct Alloc {
+        void* p;
+        size_t bytes;
+    };
+    std::vector<Alloc> allocs;
+    size_t alloc_bytes = 0, alloc_most = ~(size_t)0;      // sum over allocs, its limit (EMS_DEVICE_BYTES)
 
     // excitation: entries grouped per (component, cell), each group in list order
     struct Exc {
@@ -3906,11 +3917,19 @@ struct ems_engine {
     int alloc(T** p, size_t n)
     {
         void* q = nullptr;
-        hipError_t e = hipMalloc(&q, std::max<size_t>(n, 1) * sizeof(T));
+        const size_t bytes = std::max<size_t>(n, 1) * sizeof(T);
+        hipError_t e = device_malloc(this, &q, bytes);
         if (e != hipSuccess) return fail(EMS_E_NOMEM, std::string("hipMalloc failed: ") + hipGetErrorString(e));
-        allocs.push_back(q);
+        allocs.push_back(Alloc{q, bytes});
+        alloc_bytes += bytes;
         *p = (T*)q;
         return 0;
+    }
+    void release(size_t k)
+    {
+        (void)hipFree(allocs[k].p);
+        alloc_bytes -= allocs[k].bytes;
+        allocs.erase(allocs.begin() + (std::ptrdiff_t)k);
     }
     unsigned long long lin(unsigned x, unsigned y, unsigned z) const
     {
@@ -4069,6 +4088,7 @@ int ems_create_layout(ems_engine** out, const unsigned numLines[3], const float*
     // fields larger than the last-level cache (256 MB on MI355X) stream through it
     h->nt_fields = 2ull * 3ull * h->cs * sizeof(float) > (192ull << 20);
     if (const char* nt = std::getenv("EMS_NT_FIELDS")) h->nt_fields = std::atoi(nt) != 0;
+    if (const char* db = std::getenv("EMS_DEVICE_BYTES")) h->alloc_most = (size_t)std::strtoull(db, nullptr, 10);
     if (const char* qe = std::getenv("EMS_QUAD")) h->quad_req = std::atoi(qe) ? -1 : 0;
     if (const char* gc = std::getenv("EMS_GRAPH_CHUNK")) {
         const int v = std::atoi(gc);
@@ -5125,7 +5145,7 @@ static const void* pair_kernel(const ems_engine* h, bool lt)
 // 64^3, 34.5 -> 17.3 us at 140^3, 96 -> 57 us at 253 x 209 x 178 (plain
 // accesses; 170 us as it ran).
 constexpr unsigned long long kPairUpmlCells = 1000000;
-static int setup_pair(ems_engine* h)
+static int build_pair(ems_engine* h)
 {
     h->pair = false;
     const unsigned* N = h->N;
@@ -5247,6 +5267,19 @@ static int setup_pair(ems_engine* h)
     h->numts_alt = h->numts_dev + 2;
     h->V_base = h->V;
     h->pair = true;
+    return 0;
+}
+
+// what was free may have been taken meanwhile: single steps then
+static int setup_pair(ems_engine* h)
+{
+    const size_t n = h->allocs.size();
+    const int rc = build_pair(h);
+    if (rc != EMS_E_NOMEM) return rc;
+    while (h->allocs.size() > n) h->release(h->allocs.size() - 1);
+    if (!h->fused) h->V_alt = h->I_alt = nullptr;
+    h->flux_alt[0] = h->flux_alt[1] = nullptr;
+    h->pargs = PairArgs{};
     return 0;
 }
 
@@ -6220,16 +6253,29 @@ static void leave_pairs(ems_engine* h)
     drop_graphs(h);
     h->pair = false;
     auto release = [&](float*& p) {
-        if (!p) return;
-        h->allocs.erase(std::find(h->allocs.begin(), h->allocs.end(), (void*)p));
-        (void)hipFree(p);
-        p = nullptr;
+        for (size_t k = 0; p && k < h->allocs.size(); ++k)
+            if (h->allocs[k].p == p) {
+                h->release(k);
+                p = nullptr;
+            }
     };
     if (!h->fused) {             // the quad sweep's second fields stay
         release(h->V_alt);
         release(h->I_alt);
     }
     for (float*& f : h->flux_alt) release(f);
+}
+
+static hipError_t device_malloc(ems_engine* h, void** q, size_t bytes)
+{
+    for (;;) {
+        const bool fits = h->alloc_bytes <= h->alloc_most && bytes <= h->alloc_most - h->alloc_bytes;
+        const hipError_t e = fits ? hipMalloc(q, bytes) : hipErrorOutOfMemory;
+        if (e == hipSuccess) return e;
+        (void)hipGetLastError();
+        if (!h->pair) return e;
+        leave_pairs(h);
+    }
 }
 
 // the next one or two of at most `left` timesteps, and their samples: two in
@@ -6704,7 +6750,7 @@ void ems_destroy(ems_engine* h)
         if (G.exec) hipGraphExecDestroy(G.exec);
         if (G.graph) hipGraphDestroy(G.graph);
     }
-    for (void* p : h->allocs) hipFree(p);
+    for (const auto& a : h->allocs) hipFree(a.p);
     if (h->read_buf) hipFree(h->read_buf);
     if (h->ev0) hipEventDestroy(h->ev0);
     if (h->ev1) hipEventDestroy(h->ev1);
@@ -7458,7 +7504,7 @@ struct ems_adjoint {
     int alloc(T** p, size_t n)
     {
         void* q = nullptr;
-        hipError_t e = hipMalloc(&q, std::max<size_t>(n, 1) * sizeof(T));
+        hipError_t e = device_malloc(h, &q, std::max<size_t>(n, 1) * sizeof(T));
         if (e != hipSuccess) return fail(EMS_E_NOMEM, std::string("hipMalloc failed: ") + hipGetErrorString(e));
         allocs.push_back(q);
         *p = (T*)q;
@@ -7526,8 +7572,8 @@ int adj_reserve(ems_adjoint* a, unsigned nsteps)
     auto grow = [&](size_t n) {
         if (a->rec_steps >= n) return true;
         release();
-        if (hipMalloc((void**)&a->hc, n * step) != hipSuccess || hipMalloc((void**)&a->hv, n * step) != hipSuccess) {
-            (void)hipGetLastError();
+        if (device_malloc(a->h, (void**)&a->hc, n * step) != hipSuccess ||
+            device_malloc(a->h, (void**)&a->hv, n * step) != hipSuccess) {
             release();
             return false;
         }

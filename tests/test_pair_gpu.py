@@ -12,6 +12,7 @@ import pytest
 from oracle.operator_ref import RefOperator
 from oracle.oracle import RefEngine
 from openems_amd import scenes
+from openems_amd._native import NativeError
 from openems_amd.engine import EngineHIP
 from openems_amd.operator import Operator
 from openems_amd.simulation import Simulation
@@ -149,5 +150,48 @@ def test_sheet_source_over_many_tiles(gpu, monkeypatch):
     eng.IterateTS(7)
     assert np.max(np.abs(half.get_volt())) > 0
     assert np.array_equal(eng.get_volt(), half.get_volt()) and np.array_equal(eng.get_curr(), half.get_curr())
+    eng.close()
+    half.close()
+
+
+@pytest.mark.parametrize("pml,few,most,samples", [(False, 8, 12, 2), (True, 15, 26, 3)])
+def test_pairs_make_room(gpu, monkeypatch, pml, few, most, samples):
+    """Device memory asked for after set-up is taken from the buffers that only
+    pairs need, in the middle of a run; an engine short of it from the start
+    has no pairs.  Limits in MB: fields 4.6 (with UPML 9.9 and fluxes), as much
+    again for pairs, dump samples of 2.3 (3.1)."""
+    monkeypatch.setenv("EMS_PAIR", "1")
+    op = Operator(_graded(64, 8) if pml else _cavity(64, 60, 50))
+    last = [n - 1 for n in op.N]
+    print("case pairs make room, UPML", pml, flush=True)
+
+    def dump(e, capacity):
+        return e.add_td_dump((0, 0, 0), last, 4, capacity=capacity)
+
+    half = EngineHIP(op, fused=False)
+    half.IterateTS(2)
+    hid, box = dump(half, samples)
+    half.IterateTS(11)
+    want = half.get_volt(), half.get_curr(), half.td_dump_results(hid, box)
+    monkeypatch.setenv("EMS_DEVICE_BYTES", str(few * 1000000))
+    eng = EngineHIP(op)
+    assert eng.pair()[0] == 0
+    eng.IterateTS(13)
+    assert np.array_equal(eng.get_volt(), want[0]) and np.array_equal(eng.get_curr(), want[1])
+    eng.close()
+    monkeypatch.setenv("EMS_DEVICE_BYTES", str(most * 1000000))
+    eng = EngineHIP(op)
+    eng.set_graph(2)
+    eng.IterateTS(2)
+    assert eng.pair()[0] == 1 and eng.pair()[2] == 1
+    did, box = dump(eng, samples)
+    assert eng.pair()[0] == 0
+    with pytest.raises(NativeError, match="hipMalloc"):
+        dump(eng, 5)
+    eng.IterateTS(11)
+    assert np.max(np.abs(want[0])) > 0
+    assert np.array_equal(eng.get_volt(), want[0]) and np.array_equal(eng.get_curr(), want[1])
+    for a, b in zip(eng.td_dump_results(did, box), want[2]):
+        assert np.array_equal(a, b)
     eng.close()
     half.close()
