@@ -3733,7 +3733,7 @@ void parallel_rows(size_t n, const std::function<void(size_t, size_t)>& fn);
 struct ems_engine;
 
 // Device memory for engine h or what works on it.  Where there is none left,
-// the buffers that only pairs of timesteps need make room.
+// the read-out's buffer and the ones that only pairs of timesteps need make room.
 static hipError_t device_malloc(ems_engine* h, void** q, size_t bytes);
 
 struct ems_engine {
@@ -3762,7 +3762,8 @@ struct ems_engine {
         size_t bytes;
     };
     std::vector<Alloc> allocs;
-    size_t alloc_bytes = 0, alloc_most = ~(size_t)0;      // sum over allocs, its limit (EMS_DEVICE_BYTES)
+    size_t alloc_bytes = 0, alloc_most = ~(size_t)0;      // device memory in use, its limit (EMS_DEVICE_BYTES)
+    bool room(size_t bytes) const { return alloc_bytes <= alloc_most && bytes <= alloc_most - alloc_bytes; }
 
     // excitation: entries grouped per (component, cell), each group in list order
     struct Exc {
@@ -3883,7 +3884,7 @@ struct ems_engine {
     bool sampled0 = false;          // the samples due before the first step were taken
 
     double* energy_part = nullptr;
-    unsigned read_rows = 0;         // x planes that read_buf holds
+    size_t read_rows = 0;           // x planes that read_buf holds
     float* read_buf = nullptr;      // of get_field; not in allocs, whose growth drops the captured chunks
     std::mutex read_mu;             // the read-out that uses it
 
@@ -3924,6 +3925,15 @@ struct ems_engine {
         alloc_bytes += bytes;
         *p = (T*)q;
         return 0;
+    }
+    bool drop_read_buf()
+    {
+        std::lock_guard<std::mutex> lk(read_mu);
+        if (!read_buf) return false;
+        (void)hipFree(read_buf);
+        alloc_bytes -= read_rows * N[1] * N[2] * sizeof(float);
+        read_buf = nullptr;
+        return true;
     }
     void release(size_t k)
     {
@@ -6269,10 +6279,10 @@ static void leave_pairs(ems_engine* h)
 static hipError_t device_malloc(ems_engine* h, void** q, size_t bytes)
 {
     for (;;) {
-        const bool fits = h->alloc_bytes <= h->alloc_most && bytes <= h->alloc_most - h->alloc_bytes;
-        const hipError_t e = fits ? hipMalloc(q, bytes) : hipErrorOutOfMemory;
+        const hipError_t e = h->room(bytes) ? hipMalloc(q, bytes) : hipErrorOutOfMemory;
         if (e == hipSuccess) return e;
         (void)hipGetLastError();
+        if (h->drop_read_buf()) continue;
         if (!h->pair) return e;
         leave_pairs(h);
     }
@@ -6532,6 +6542,25 @@ int ems_sync(ems_engine* h)
 
 constexpr size_t kReadBytes = 64u << 20;      // device buffer of a field read-out
 
+// a field through host memory, a component at a time
+static int get_field_staged(const ems_engine* h, const float* d, float* out)
+{
+    const unsigned* N = h->N;
+    const size_t Nx = N[0], Ny = N[1], Nz = N[2];
+    std::vector<float> stage(Nx * Ny * Nz);
+    for (unsigned c = 0; c < 3; ++c) {
+        HIPCHK(hipMemcpy(stage.data(), d + c * h->cs, stage.size() * sizeof(float), hipMemcpyDeviceToHost));
+        parallel_rows(Nx * Ny, [&](size_t a, size_t b) {
+            for (size_t r = a; r < b; ++r) {
+                const float* q = stage.data() + r / Ny + Nx * (r % Ny);
+                float* o = out + (c * Nx * Ny + r) * Nz;
+                for (size_t z = 0; z < Nz; ++z) o[z] = q[z * Nx * Ny];
+            }
+        });
+    }
+    return 0;
+}
+
 static int get_field(ems_engine* h, const float* d, float* out)
 {
     if (!h || !out) return fail(EMS_E_ARG, "null argument");
@@ -6540,27 +6569,34 @@ static int get_field(ems_engine* h, const float* d, float* out)
     // turned on the device, kReadBytes at a time; several threads may read at once
     std::lock_guard<std::mutex> lk(h->read_mu);
     const unsigned *N = h->N;
-    const size_t row = (size_t)N[1] * N[2];              // floats of one x
+    const size_t row = (size_t)N[1] * N[2], rows = 3 * (size_t)N[0];     // floats of one x plane, planes of all components
     if (!h->read_buf) {
-        unsigned n = (unsigned)std::min<size_t>(N[0], std::max<size_t>(1, kReadBytes / (row * sizeof(float))));
-        while (hipMalloc((void**)&h->read_buf, n * row * sizeof(float)) != hipSuccess) {
+        // as many planes as the device has room for; with none, through the host
+        size_t n = std::min(rows, std::max<size_t>(1, kReadBytes / (row * sizeof(float))));
+        for (; n; n /= 2) {
+            if (h->room(n * row * sizeof(float)) &&
+                hipMalloc((void**)&h->read_buf, n * row * sizeof(float)) == hipSuccess) break;
             (void)hipGetLastError();
             h->read_buf = nullptr;
-            if (n == 1) return fail(EMS_E_NOMEM, "no device memory for the field read-out");
-            n /= 2;
         }
+        if (!n) return get_field_staged(h, d, out);
         h->read_rows = n;
+        h->alloc_bytes += n * row * sizeof(float);
     }
-    const unsigned most = h->read_rows;
-    for (unsigned c = 0; c < 3; ++c)
-        for (unsigned x0 = 0; x0 < N[0]; x0 += most) {
-            const unsigned nx = std::min(most, N[0] - x0);
-            hipLaunchKernelGGL(k_to_nijk, dim3((nx + kTurn - 1) / kTurn, (N[2] + kTurn - 1) / kTurn, std::min(N[1], 65535u)), dim3(kTurn * 8),
-                               0, h->stream, d + c * h->cs, h->read_buf, N[0], N[1], N[2], x0, nx);
-            HIPCHK(hipGetLastError());
-            HIPCHK(hipMemcpyAsync(out + ((size_t)c * N[0] + x0) * row, h->read_buf, nx * row * sizeof(float),
-                                  hipMemcpyDeviceToHost, h->stream));
+    for (size_t r0 = 0; r0 < rows; r0 += h->read_rows) {
+        const size_t r1 = std::min(rows, r0 + h->read_rows);
+        for (size_t r = r0; r < r1;) {
+            const unsigned c = (unsigned)(r / N[0]), x0 = (unsigned)(r % N[0]);
+            const unsigned nx = (unsigned)std::min<size_t>(N[0] - x0, r1 - r);
+            hipLaunchKernelGGL(k_to_nijk, dim3((nx + kTurn - 1) / kTurn, (N[2] + kTurn - 1) / kTurn, std::min(N[1], 65535u)),
+                               dim3(kTurn * 8), 0, h->stream, d + c * h->cs, h->read_buf + (r - r0) * row, N[0], N[1], N[2],
+                               x0, nx);
+            r += nx;
         }
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipMemcpyAsync(out + r0 * row, h->read_buf, (r1 - r0) * row * sizeof(float), hipMemcpyDeviceToHost,
+                              h->stream));
+    }
     HIPCHK(hipStreamSynchronize(h->stream));
     return 0;
 }

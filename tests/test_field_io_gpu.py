@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 from openems_amd import scenes
+from openems_amd._native import NativeError
 from openems_amd.engine import EngineHIP
 from openems_amd.operator import Operator
 
@@ -113,3 +114,40 @@ def test_fields_read_by_several_threads(gpu):
             t.join()
         eng.close()
     assert not bad
+
+
+def test_fields_read_with_little_device_memory(gpu, monkeypatch):
+    """The read-out's device buffer holds all planes, two of 81 (blocks across
+    components), or nothing; a later allocation takes it back."""
+    op = Operator(dict(scenes.pec_cavity(8, 10), lines=[np.arange(n, dtype=np.float64) for n in (27, 11, 33)], probes=[]))
+    rng = np.random.default_rng(3)
+    want = [rng.standard_normal((3,) + tuple(op.N)).astype(np.float32) for _ in range(2)]
+    print("case fields read with little memory", flush=True)
+
+    def engine(limit):
+        monkeypatch.setenv("EMS_DEVICE_BYTES", str(limit))
+        try:
+            return EngineHIP(op, fused=False)
+        except NativeError:
+            return None
+
+    lo, hi = 0, 1 << 24            # the least memory that the engine itself needs
+    while hi - lo > 256:
+        mid = (lo + hi) // 2
+        eng = engine(mid)
+        if eng is None:
+            lo = mid
+        else:
+            hi = mid
+            eng.close()
+    plane = 4 * 11 * 33
+    for extra in (0, 2 * plane, 1 << 24):
+        eng = engine(hi + extra)
+        eng.set_volt(want[0])
+        eng.set_curr(want[1])
+        for _ in range(2):
+            assert np.array_equal(eng.get_volt(), want[0]) and np.array_equal(eng.get_curr(), want[1])
+        if extra == 1 << 24:       # more than is left beside the buffer
+            eng.add_td_dump((0, 0, 0), (26, 10, 32), 1, capacity=((1 << 24) - 20000) // (12 * 27 * 11 * 33))
+            assert np.array_equal(eng.get_volt(), want[0])
+        eng.close()
