@@ -5302,25 +5302,79 @@ namespace {
 
 struct HookPlan {
     HookJob d{};
-    std::vector<unsigned long long> cells;    // sorted component * cs + cell of a list job
+    std::vector<unsigned long long> elems;    // sorted component * cs + cell of a list job
+    std::vector<unsigned> cells;              // sorted cells that a list job sets all components of
     std::vector<unsigned char> lines[3];      // per axis and line: bit c where component c has such an element
     bool writes = true;                       // it sets field elements
     const ems_engine::MurGeo* mur = nullptr;  // a Mur face's job
     int face = -1;
 };
 
+// stable sort by the bits from `lo` on.  Lists of a mesh's cells have millions
+// of entries in any order: 4 million keys 27 ms, std::sort 183
+void sort_keys(std::vector<unsigned long long>& a, unsigned lo = 0)
+{
+    constexpr unsigned kBits = 12, kBuckets = 1u << kBits;
+    auto less = [lo](unsigned long long l, unsigned long long r) { return l >> lo < r >> lo; };
+    if (std::is_sorted(a.begin(), a.end(), less)) return;
+    if (a.size() < 4 * kBuckets) {
+        std::stable_sort(a.begin(), a.end(), less);
+        return;
+    }
+    const unsigned long long top = *std::max_element(a.begin(), a.end());
+    std::vector<unsigned long long> b(a.size());
+    for (unsigned s = lo; s < 64 && top >> s; s += kBits) {
+        size_t at[kBuckets + 1] = {};
+        for (unsigned long long k : a) ++at[(k >> s & (kBuckets - 1)) + 1];
+        for (unsigned d = 0; d < kBuckets; ++d) at[d + 1] += at[d];
+        for (unsigned long long k : a) b[at[k >> s & (kBuckets - 1)]++] = k;
+        a.swap(b);
+    }
+}
+
 // the lines that a list job's elements lie on
 void find_lines(const ems_engine* h, HookPlan& q)
 {
     for (int n = 0; n < 3; ++n) q.lines[n].assign(h->N[n], 0);
-    for (unsigned long long e : q.cells) {
+    auto mark = [&](unsigned p, unsigned char bits) {
+        const unsigned z = p / h->g.plane, r = p - z * h->g.plane, y = r / h->N[0];
+        q.lines[0][r - y * h->N[0]] |= bits;
+        q.lines[1][y] |= bits;
+        q.lines[2][z] |= bits;
+    };
+    for (unsigned long long e : q.elems) {
         const unsigned c = e >= 2 * h->cs ? 2u : e >= h->cs ? 1u : 0u;
-        const unsigned p = (unsigned)(e - c * h->cs), z = p / h->g.plane, r = p - z * h->g.plane, y = r / h->N[0];
-        const unsigned char bit = (unsigned char)(1u << c);
-        q.lines[0][r - y * h->N[0]] |= bit;
-        q.lines[1][y] |= bit;
-        q.lines[2][z] |= bit;
+        mark((unsigned)(e - c * h->cs), (unsigned char)(1u << c));
     }
+    for (unsigned p : q.cells) mark(p, 7);
+}
+
+// whether two list jobs share an element
+bool share_element(const ems_engine* h, const HookPlan& a, const HookPlan& b)
+{
+    for (size_t i = 0, j = 0; i < a.elems.size() && j < b.elems.size();) {
+        if (a.elems[i] == b.elems[j]) return true;
+        if (a.elems[i] < b.elems[j]) ++i;
+        else ++j;
+    }
+    auto in_cells = [h](const std::vector<unsigned long long>& e, const std::vector<unsigned>& c) {
+        if (c.size() < e.size() / 3) {
+            for (unsigned x : c)
+                for (unsigned n = 0; n < 3; ++n)
+                    if (std::binary_search(e.begin(), e.end(), n * h->cs + x)) return true;
+            return false;
+        }
+        for (unsigned long long k : e)
+            if (std::binary_search(c.begin(), c.end(), (unsigned)(k % h->cs))) return true;
+        return false;
+    };
+    if (in_cells(a.elems, b.cells) || in_cells(b.elems, a.cells)) return true;
+    for (size_t i = 0, j = 0; i < a.cells.size() && j < b.cells.size();) {
+        if (a.cells[i] == b.cells[j]) return true;
+        if (a.cells[i] < b.cells[j]) ++i;
+        else ++j;
+    }
+    return false;
 }
 
 // an element of list job l on the line that Mur job m reads (the neighbour
@@ -5354,12 +5408,7 @@ bool hooks_conflict(const ems_engine* h, const HookPlan& a, const HookPlan& b)
         return mur_touches(m, l);
     }
     if (!a.writes && !b.writes) return false;
-    for (size_t i = 0, j = 0; i < a.cells.size() && j < b.cells.size();) {
-        if (a.cells[i] == b.cells[j]) return true;
-        if (a.cells[i] < b.cells[j]) ++i;
-        else ++j;
-    }
-    return false;
+    return share_element(h, a, b);
 }
 
 }  // namespace
@@ -5457,8 +5506,8 @@ static int setup_hooks(ems_engine* h)
         q.d.length = h->sigLen;
         q.d.period = h->period;
         q.d.ts_bias = bias;
-        q.cells = e.h_glin;
-        std::sort(q.cells.begin(), q.cells.end());
+        q.elems = e.h_glin;
+        sort_keys(q.elems);
         if (!curr && nmur) find_lines(h, q);
         return q;
     };
@@ -5553,36 +5602,43 @@ static int setup_hooks(ems_engine* h)
         q.d.kind = kRlcApply;
         q.d.n = h->rlc[k].count;
         q.d.rlc = h->rlc[k];
-        q.cells = h->h_rlc[k];
-        std::sort(q.cells.begin(), q.cells.end());
+        q.elems = h->h_rlc[k];
+        sort_keys(q.elems);
         if (nmur) find_lines(h, q);
         list.push_back(q);
     }
     auto lor_apply = [&](int side, HookPlan& q) {
-        // a cell's orders in creation order
-        std::vector<std::pair<unsigned, LorTerm>> t;
+        // a cell's orders in creation order: keys of the cell and the place in the lists
+        std::vector<unsigned long long> keys;
+        std::vector<std::pair<size_t, const LorDev*>> from;       // first place of each list
+        size_t all = 0;
+        for (const auto& l : h->h_lor) all += l.size();
+        keys.reserve(all);
         for (size_t k = side; k < h->lor.size(); k += 2) {
             if (!(side ? h->lor_i : h->lor_v)[k / 2]) continue;
-            const LorDev& d = h->lor[k];
-            for (unsigned j = 0; j < d.count; ++j) t.push_back({h->h_lor[k / 2][j], LorTerm{d.ade, j, d.count}});
+            from.push_back({keys.size(), &h->lor[k]});
+            for (unsigned x : h->h_lor[k / 2]) keys.push_back((unsigned long long)x << 32 | keys.size());
         }
-        std::stable_sort(t.begin(), t.end(), [](const auto& l, const auto& r) { return l.first < r.first; });
-        std::vector<unsigned> cell, beg;
-        std::vector<LorTerm> term;
-        for (const auto& e : t) {
-            if (cell.empty() || cell.back() != e.first) {
-                cell.push_back(e.first);
-                beg.push_back((unsigned)term.size());
+        if (keys.empty()) return 0;
+        if (keys.size() > 0xFFFFFFFFull) return fail(EMS_E_ARG, "too many dispersive cells");
+        sort_keys(keys, 32);
+        std::vector<unsigned>& cell = q.cells;
+        std::vector<unsigned> beg;
+        std::vector<LorTerm> term(keys.size());
+        for (size_t t = 0; t < keys.size(); ++t) {
+            const unsigned x = (unsigned)(keys[t] >> 32), at = (unsigned)keys[t];
+            if (cell.empty() || cell.back() != x) {
+                cell.push_back(x);
+                beg.push_back((unsigned)t);
             }
-            term.push_back(e.second);
+            size_t f = from.size() - 1;
+            while (from[f].first > at) --f;
+            term[t] = LorTerm{from[f].second->ade, at - (unsigned)from[f].first, from[f].second->count};
         }
         beg.push_back((unsigned)term.size());
         q.d.kind = kLorApply;
         q.d.curr = side;
         q.d.n = 3 * (unsigned)cell.size();
-        if (!q.d.n) return 0;
-        for (int n = 0; n < 3; ++n)
-            for (unsigned x : cell) q.cells.push_back(n * h->cs + x);
         if (!side && nmur) find_lines(h, q);
         unsigned *dc, *db;
         LorTerm* dt;
@@ -5597,7 +5653,7 @@ static int setup_hooks(ems_engine* h)
     };
     HookPlan lv, li;
     if ((rc = lor_apply(0, lv)) || (rc = lor_apply(1, li))) return rc;
-    if (lv.d.n) list.push_back(lv);
+    if (lv.d.n) list.push_back(std::move(lv));
     std::vector<HookPlan> post, apply;
     for (int k = nmur - 1; k >= 0; --k) {
         post.push_back(mur_job(kMurPost, k));
@@ -5622,18 +5678,18 @@ static int setup_hooks(ems_engine* h)
         q.d.n = h->ss.n;
         q.d.ss = h->ss;
         q.writes = false;
-        q.cells = h->h_ss;
-        std::sort(q.cells.begin(), q.cells.end());
+        q.elems = h->h_ss;
+        sort_keys(q.elems);
         if (nmur) find_lines(h, q);
         ss = (int)v.size();
         v.push_back(q);
     }
-    v.insert(v.end(), list.begin(), list.end());
+    v.insert(v.end(), std::make_move_iterator(list.begin()), std::make_move_iterator(list.end()));
     v.insert(v.end(), apply.begin(), apply.end());
     if (h->exc[0].G && !h->qsrc.beg) v.push_back(exc_job(h->exc[0], 0, 0));
     // the steady-state evaluation's energy reads the voltages before any hook sets them
     if ((rc = build_hook_launches(h, v, false, h->hooks_v, ss, &h->hooks_ss))) return rc;
-    if (li.d.n) c.push_back(li);
+    if (li.d.n) c.push_back(std::move(li));
     if (h->exc[1].G) c.push_back(exc_job(h->exc[1], 1, -1));
     return build_hook_launches(h, c, false, h->hooks_i);
 }
@@ -5682,6 +5738,7 @@ int ems_init(ems_engine* h)
     if ((rc = setup_vsrc(h))) return rc;
     if ((rc = setup_pair(h))) return rc;
     if ((rc = setup_hooks(h))) return rc;
+    h->h_lor = {};               // of the set-up only, four bytes a dispersive cell
     // ems_energy's partial sums: allocated later, they would drop the captured chunks
     if (!h->energy_part && (rc = h->alloc(&h->energy_part, 2 * kEnergyBlocks))) return rc;
     // small compressed tables (both half steps' within 32 KiB) go to LDS in the quad kernels

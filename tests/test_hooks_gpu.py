@@ -69,6 +69,43 @@ def test_hooks_match_oracle(gpu, name, make, steady):
     e.close()
 
 
+@pytest.mark.parametrize("mur", [False, True])
+def test_long_unordered_ade_lists(gpu, mur):
+    """Three orders over most cells of the mesh (faces included), in random
+    order and overlapping, with lumped elements among them: lists long enough
+    for the counting sort, against the oracle."""
+    scene = dict(scenes.mur_layers(40, 36, 30, 60), bc=[2] * 6) if mur else scenes.upml_bricks(40, 60, nbricks=6, dump=False)
+    print("case hooks long ADE lists, Mur", mur, flush=True)
+    op = Operator(scene)
+    rng = np.random.default_rng(8)
+    cells = int(np.prod(op.N))
+    lor = []
+    for share, lorentz, curr in ((0.7, True, True), (0.5, False, True), (0.02, False, False)):
+        at = rng.permutation(cells)[:int(share * cells)]
+        k = len(at)
+        o = {"pos": np.stack(np.unravel_index(at, tuple(op.N))).astype(np.uint32), "volt": True, "curr": curr}
+        for s in "vi":
+            o[s + "_int"] = rng.uniform(0.8, 0.95, (3, k)).astype(np.float32)
+            o[s + "_ext"] = rng.uniform(1e-3, 5e-3, (3, k)).astype(np.float32)
+            o[s + "_lor"] = rng.uniform(1e-3, 5e-3, (3, k)).astype(np.float32) if lorentz else None
+        lor.append(o)
+    assert lor[0]["pos"].shape[1] > 16384 and lor[2]["pos"].shape[1] < 16384
+    rlc = {"pos": np.stack([rng.choice(np.arange(3, n - 3), 6, replace=False) for n in op.N]).astype(np.uint32),
+           "dir": rng.integers(0, 3, 6).astype(np.int32)}
+    for name in ("i2v", "ilv", "vvd", "vv2", "vj1", "vj2", "ib0", "b1", "b2"):
+        rlc[name] = rng.uniform(0.5, 0.9, 6).astype(np.float32) if name == "vvd" else rng.uniform(-0.05, 0.05, 6).astype(np.float32)
+    eng = EngineHIP(op, fused=False, lorentz=lor, rlc=rlc)
+    eng.IterateTS(60)
+    ref = RefEngine(RefOperator(scene).build(), "basic", lorentz=lor, rlc=rlc)
+    ref.iterate(60)
+    rv, rc = ref.raw_views()
+    assert np.max(np.abs(rv)) > 0
+    assert np.array_equal(eng.get_volt(), rv)
+    assert np.array_equal(eng.get_curr(), rc)
+    eng.close()
+    ref.close()
+
+
 def _sweep_mur(nx, faces=(2, 2, 2, 2, 2, 2)):
     return lambda: dict(scenes.mur_layers(nx, 26, 22, 120), bc=list(faces))
 
