@@ -7799,6 +7799,7 @@ int ems_adj_forward(ems_adjoint* a, unsigned nsteps, double* J)
     ems_engine* h = a->h;
     HIPCHK(hipSetDevice(h->device));
     int rc;
+    a->forward_done = false;     // until this run is: its records and saved states replace the last one's
     if ((rc = sync_probe_tables(h))) return rc;
     HIPCHK(hipStreamSynchronize(h->stream));
     HIPCHK(hipMemsetAsync(a->d_F, 0, 2 * a->np * sizeof(double), h->stream));

@@ -1,10 +1,13 @@
 """Adjoint gradients (include/ems_hip.h ems_adj_*, openems_amd.adjoint)
 against centred finite differences of the oracle's float64 engine on the
 same operator: the reference gradient in double precision on the CPU."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 from openems_amd import scenes
+from openems_amd._native import NativeError, check, dp, lib
 from openems_amd.adjoint import DesignProblem, objective
 from oracle.operator_ref import RefOperator
 from oracle.oracle import RefEngine
@@ -198,3 +201,35 @@ def test_kept_records_equal_replayed_segments(gpu, monkeypatch, steps, every):
     for a, b in zip(*out):
         assert np.array_equal(a, b)
     assert np.abs(out[0][1]).max() > 0
+
+
+def _forward_backward(prob, steps):
+    """One run on the problem's handle: objective, gradient of the operator's coefficients, the engine's fields and step."""
+    J = C.c_double()
+    check(lib().ems_adj_forward(prob._adj, steps, C.byref(J)))
+    g = np.zeros((2, 3 * int(np.prod(prob.box_hi - prob.box_lo + 1))))
+    check(lib().ems_adj_backward(prob._adj, g[0].ctypes.data_as(dp), g[1].ctypes.data_as(dp)))
+    return np.array(J.value), g, prob._eng.get_volt(), prob._eng.get_curr(), np.array(prob._eng.numTS)
+
+
+def test_backward_after_a_failed_forward_is_refused(gpu, monkeypatch):
+    """A forward run that finds no memory for its records leaves nothing to run
+    backwards; the next one that does is as without it."""
+    scene, probes, freq = _small()
+    eps = scene["materials"][0]["grid"]["eps"].copy()
+    monkeypatch.setenv("EMS_DEVICE_BYTES", str(64 << 20))
+    out = []
+    for fail in (False, True):
+        print("case adjoint, a forward run fails:", fail, flush=True)
+        prob = DesignProblem(scene, probes, freq, 200, checkpoint_every=10 ** 6)
+        prob.forward(eps)
+        if fail:
+            with pytest.raises(NativeError, match="no device memory"):
+                check(lib().ems_adj_forward(prob._adj, 10 ** 6, None))
+            with pytest.raises(NativeError, match="ems_adj_forward first"):
+                check(lib().ems_adj_backward(prob._adj, None, None))
+        out.append(_forward_backward(prob, 60))
+        prob.close()
+    assert np.abs(out[0][1]).max() > 0
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
