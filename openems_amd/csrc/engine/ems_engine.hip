@@ -2098,6 +2098,7 @@ __global__ __launch_bounds__(kBlock, 3) void k_step4t(const Step4Args ag, const 
 // ---------------------------------------------------------------------------
 constexpr unsigned kPairMax = 1024;      // threads of a workgroup (columns of its tile)
 constexpr unsigned kPairMaxPml = 512;    // with UPML, whose fluxes and coefficients take 40 registers more
+constexpr unsigned kLdsBytes = 160u * 1024u;   // of a CU
 constexpr unsigned kPairLds = 18;        // floats of LDS per column: 3 fields x 3 components x 2 planes
 
 // UPML of k_pair: the slab table in device memory, both sides' arrays
@@ -5102,8 +5103,8 @@ static void choose_pair_tile(const unsigned N[3], const PairCost& cost, unsigned
             lty = ty;
             const unsigned T = (tx * ty + 63u) / 64u * 64u;
             const size_t lds = (size_t)column * T + table;
-            if (T > most || lds > 160u * 1024u) continue;
-            const unsigned res = std::min(waves / (T / 64u), (unsigned)(160u * 1024u / lds));
+            if (T > most || lds > kLdsBytes) continue;
+            const unsigned res = std::min(waves / (T / 64u), (unsigned)(kLdsBytes / lds));
             if (!res) continue;
             unsigned last = 0;
             for (unsigned nz = 1; nz <= N[2]; ++nz) {
@@ -5212,7 +5213,8 @@ static int build_pair(ems_engine* h)
     h->pair_threads = (a.tx * a.ty + 63u) / 64u * 64u;
     h->pair_blocks = a.ntiles * ((N[2] + a.zd - 1) / a.zd);
     h->pair_lds = (size_t)lds * h->pair_threads + table;
-    HIPCHK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->pair_lds));
+    // a limit of the kernel, not of this engine: engines of other tiles share it
+    HIPCHK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes));
     // sources: lists per column ordered by plane, their planes, and the tiles
     // (rims included) that hold one
     std::vector<unsigned> mask((a.ntiles + 31) / 32, 0u);

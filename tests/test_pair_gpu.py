@@ -195,3 +195,28 @@ def test_pairs_make_room(gpu, monkeypatch, pml, few, most, samples):
         assert np.array_equal(a, b)
     eng.close()
     half.close()
+
+
+def test_engines_of_different_tiles_in_turn(gpu, monkeypatch):
+    """An engine whose tiles take 72 KB of LDS goes on beside one made later
+    whose tiles take 5 KB, direct launches and replayed chunks."""
+    monkeypatch.setenv("EMS_PAIR", "1")
+    op = Operator(_cavity(70, 40, 20, True))
+    half = EngineHIP(op, fused=False)
+    half.IterateTS(40)
+    engs = []
+    for tile in ("64,16,5", "64,16,20", "8,8,4"):
+        monkeypatch.setenv("EMS_PAIR_TILE", tile)
+        engs.append(EngineHIP(op))
+        assert engs[-1].pair()[1] == tuple(int(k) for k in tile.split(","))
+    print("case pairs of three tiles in turn", flush=True)
+    for e in engs:
+        e.set_graph(6)
+    for n in (4, 1, 15, 20):
+        for e in engs:
+            e.IterateTS(n)
+    for e in engs:
+        assert np.array_equal(e.get_volt(), half.get_volt()) and np.array_equal(e.get_curr(), half.get_curr())
+        e.close()
+    assert np.max(np.abs(half.get_volt())) > 0
+    half.close()
