@@ -220,3 +220,48 @@ def test_engines_of_different_tiles_in_turn(gpu, monkeypatch):
         e.close()
     assert np.max(np.abs(half.get_volt())) > 0
     half.close()
+
+
+@pytest.mark.parametrize("graph", [0, 6, 9])
+@pytest.mark.parametrize("shape,interval,curr", [((260, 12, 10), 0, False), ((256, 17, 9), 3, True), ((264, 10, 21), 5, False)])
+def test_pairs_beside_quad_sweeps(gpu, monkeypatch, shape, interval, curr, graph):
+    """On rows of 64 quads the single steps between pairs are the quad sweep's,
+    which swaps the field buffers and not the counters and writes no last
+    line: from random fields, against the half steps and the oracle."""
+    monkeypatch.delenv("EMS_PAIR", raising=False)
+    scene = _cavity(*shape, curr)
+    print("case pairs beside quad sweeps", shape, interval, graph, flush=True)
+    op = Operator(scene)
+    ref = RefEngine(RefOperator(scene).build(), "basic")
+    ref.iterate(41)
+    rv, rc = ref.raw_views()
+    rng = np.random.default_rng(9)
+    v = rng.standard_normal((3,) + tuple(op.N)).astype(np.float32)
+    c = rng.standard_normal((3,) + tuple(op.N)).astype(np.float32)
+    out = []
+    for fused in (None, False):
+        eng = EngineHIP(op, fused=fused)
+        assert eng.pair()[0] == (fused is None) and (eng.fused()[0] == 3) == (fused is None)
+        eng.set_graph(graph)
+        if interval:
+            pos = np.repeat(np.array([[k // 2] for k in shape], np.uint32), 3, 1)
+            pid = eng.add_probe(2, [0, 1, 2], pos, None, [1.0] * 3, interval, 0, 0, 10 ** 6, 400)
+        eng.IterateTS(5)
+        eng.IterateTS(36)
+        assert np.array_equal(eng.get_volt(), rv) and np.array_equal(eng.get_curr(), rc)
+        for n in (41, 7, 30, 90):
+            eng.set_volt(v)
+            eng.set_curr(c)
+            eng.IterateTS(n)
+            out.append((eng.get_volt(), eng.get_curr()))
+        if interval:
+            out.append(eng.probe_results(pid))
+        if fused is None:
+            assert eng.pair()[2] > 0
+            if graph:
+                assert eng.graph()[2] > 0
+        eng.close()
+    ref.close()
+    half = len(out) // 2
+    for a, b in zip(out[:half], out[half:]):
+        assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
