@@ -407,11 +407,14 @@ void ems_batch_destroy(ems_batch* b);
  * timestep (two half steps with UPML and sources) for the objective
  *   J = sum_p |F_p|^2,  F_p = sum_{n=1..N} (V[comp_p](pos_p) / divisor_p)(n) exp(-2 pi i f n dT) dT
  * (V after step n, N steps from the engine's state at ems_adj_forward).
- * ems_adj_forward runs the N steps, saving the state every checkpoint_every
- * steps; ems_adj_backward replays each segment from its checkpoint and runs
- * the transposed half steps backwards in time, accumulating dJ/dvi and dJ/dvv
- * (double, [3][box]) on the edges of the inclusive sensitivity box
- * box_lo..box_hi, which must not overlap the UPML.  The engine runs two half
+ * ems_adj_forward runs the N steps and keeps, of every step, what the reverse
+ * run needs of the sensitivity box, where that takes at most an eighth of the
+ * free device memory; else it saves the state every checkpoint_every steps,
+ * and ems_adj_backward replays each segment from its checkpoint first.
+ * ems_adj_backward runs the transposed half steps backwards in time,
+ * accumulating dJ/dvi and dJ/dvv (double, [3][box]) on the edges of the
+ * inclusive sensitivity box box_lo..box_hi, which must not overlap the UPML.
+ * A forward run that fails leaves nothing to run backwards.  The engine runs two half
  * steps and carries no Mur, Lorentz or lumped RLC; its probes and dumps are
  * not sampled during these runs.  Afterwards the engine holds the state at
  * the end of the forward run. */
@@ -421,6 +424,9 @@ int ems_adj_create(ems_adjoint** out, ems_engine* h, unsigned nprobe, const unsi
                    unsigned checkpoint_every);
 int ems_adj_forward(ems_adjoint* a, unsigned nsteps, double* J);
 int ems_adj_backward(ems_adjoint* a, double* dJ_dvi, double* dJ_dvv);
+/* kept: 1 when the last forward run kept every step's record; steps: the steps
+ * that the record buffers hold */
+int ems_adj_get_records(const ems_adjoint* a, int* kept, unsigned long long* steps);
 void ems_adj_destroy(ems_adjoint* a);
 
 #ifdef __cplusplus

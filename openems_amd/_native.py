@@ -147,6 +147,7 @@ ENGINE_API = [
     ("ems_adj_create", C.c_int, [C.POINTER(vp), vp, C.c_uint, up, up, dp, C.c_double, C.c_double, up, up, C.c_uint]),
     ("ems_adj_forward", C.c_int, [vp, C.c_uint, dp]),
     ("ems_adj_backward", C.c_int, [vp, dp, dp]),
+    ("ems_adj_get_records", C.c_int, [vp, ip, C.POINTER(C.c_ulonglong)]),
     ("ems_adj_destroy", None, [vp]),
 ]
 

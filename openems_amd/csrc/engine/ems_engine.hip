@@ -7866,7 +7866,7 @@ int ems_adj_backward(ems_adjoint* a, double* dJ_dvi, double* dJ_dvv)
             for (unsigned j = 0; j < len; ++j) {
                 adj_sample(a, (int)j, false);
                 bool ahead = false;
-            rc = launch_step(h, nullptr, false, ahead);
+                rc = launch_step(h, nullptr, false, ahead);
                 ++h->numTS;
                 if (rc) return rc;
             }
@@ -7882,6 +7882,14 @@ int ems_adj_backward(ems_adjoint* a, double* dJ_dvi, double* dJ_dvv)
     if ((rc = adj_restore(a, a->ck[S]))) return rc;
     if (dJ_dvi) HIPCHK(hipMemcpy(dJ_dvi, a->gvi, 3 * a->box.n * sizeof(double), hipMemcpyDeviceToHost));
     if (dJ_dvv) HIPCHK(hipMemcpy(dJ_dvv, a->gvv, 3 * a->box.n * sizeof(double), hipMemcpyDeviceToHost));
+    return 0;
+}
+
+int ems_adj_get_records(const ems_adjoint* a, int* kept, unsigned long long* steps)
+{
+    if (!a) return fail(EMS_E_ARG, "null adjoint");
+    if (kept) *kept = a->kept ? 1 : 0;
+    if (steps) *steps = a->rec_steps;
     return 0;
 }
 

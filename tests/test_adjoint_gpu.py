@@ -184,11 +184,16 @@ def test_full_size_directional_derivative(gpu):
     assert abs(ad - fd) <= 1e-3 * abs(fd)
 
 
+def _records(prob):
+    kept, steps = C.c_int(), C.c_ulonglong()
+    check(lib().ems_adj_get_records(prob._adj, C.byref(kept), C.byref(steps)))
+    return kept.value, steps.value
+
+
 @pytest.mark.parametrize("steps,every", [(1, 8), (37, 8), (64, 64)])
 def test_kept_records_equal_replayed_segments(gpu, monkeypatch, steps, every):
     """The gradient from records kept during the forward run equals the one
-    from replayed segments bit for bit, also after a second, longer run, and
-    the engine ends at the same state."""
+    from replayed segments bit for bit, and the engine ends at the same state."""
     scene, probes, freq = _small()
     eps = scene["materials"][0]["grid"]["eps"].copy()
     out = []
@@ -197,6 +202,7 @@ def test_kept_records_equal_replayed_segments(gpu, monkeypatch, steps, every):
         print("case adjoint records, keep", keep, "steps", steps, flush=True)
         prob = DesignProblem(scene, probes, freq, 200 + steps, checkpoint_every=every)
         out.append(prob.value_and_grad(eps) + (prob._eng.get_volt(), prob._eng.get_curr(), prob._eng.numTS))
+        assert _records(prob)[0] == int(keep)
         prob.close()
     for a, b in zip(*out):
         assert np.array_equal(a, b)
@@ -233,3 +239,32 @@ def test_backward_after_a_failed_forward_is_refused(gpu, monkeypatch):
     assert np.abs(out[0][1]).max() > 0
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+def test_runs_of_all_lengths_on_one_handle(gpu, monkeypatch):
+    """Runs shorter than a segment, longer and shorter ones again on one
+    handle, each kept, each replayed, or in turn: the same bits; the records
+    grow to the longest kept run (8 steps at least)."""
+    scene, probes, freq = _small()
+    eps = scene["materials"][0]["grid"]["eps"].copy()
+    lengths = (5, 37, 12, 64, 3)
+    out = []
+    for name, keeps, holds in (("kept", "11111", (200, 200, 200, 200, 200)), ("replayed", "00000", (8, 8, 8, 8, 8)),
+                               ("in turn", "01010", (8, 37, 37, 64, 64)), ("in turn", "10101", (8, 8, 12, 12, 12))):
+        print("case adjoint runs on one handle,", name, flush=True)
+        monkeypatch.setenv("EMS_ADJ_KEEP", "1" if name == "kept" else "0")
+        prob = DesignProblem(scene, probes, freq, 200, checkpoint_every=8)
+        prob.forward(eps)
+        runs = []
+        for n, keep, hold in zip(lengths, keeps, holds):
+            monkeypatch.setenv("EMS_ADJ_KEEP", keep)
+            runs.append(_forward_backward(prob, n))
+            assert _records(prob) == (int(keep), hold)
+        out.append(runs)
+        prob.close()
+    for other in out[1:]:
+        for a, b in zip(out[0], other):
+            for x, y in zip(a, b):
+                assert np.array_equal(x, y)
+    # (in the short runs nothing gets from the probes back to the box: a line a step at most)
+    assert np.abs(out[0][1][1]).max() > 0 and np.abs(out[0][3][1]).max() > 0
