@@ -295,8 +295,8 @@ def run_batched(count, steps, tune_steps=6, sequential=True):
            "autotuned": {"tile_x": cfg["tile_x"], "grid": cfg["grid"], "work_items": cfg["work_items"],
                          "groups": cfg["groups"], "group_bytes": cfg["group_bytes"], "streams": b.streams(),
                          "zdepths": sorted(set(cfg["zdepth"])), "tuned_ms_per_step": round(tuned_ms, 4)},
-           "sequential_engine": "default single engine (compressed coefficients, two half steps), one "
-                                "instance after another, setup excluded"}
+           "sequential_engine": "default single engine (compressed coefficients, two timesteps per launch from a "
+                                "million cells, else two half steps), one instance after another, setup excluded"}
     b.close()
     return out
 
