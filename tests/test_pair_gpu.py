@@ -42,6 +42,30 @@ def _sheet(nx, ny, nz):
     return s
 
 
+def _columns(nx, ny, nz):
+    """columns with one entry a plane, with a gap, with several entries on some planes, and of currents"""
+    s = _cavity(nx, ny, nz)
+    s["excitations"] = [
+        {"type": 0, "val": (0.0, 0.0, 1.0), "start": (12, 0, 0), "stop": (12, ny - 1, nz - 1)},
+        {"type": 0, "val": (0.0, 0.5, 0.0), "start": (20, 3, 2), "stop": (20, 14, 6)},
+        {"type": 0, "val": (0.0, 0.5, 0.0), "start": (20, 3, 12), "stop": (20, 14, nz - 1)},
+        {"type": 0, "val": (0.3, 0.0, 0.7), "start": (4, 8, 5), "stop": (9, 8, 16)},
+        {"type": 2, "val": (0.0, 0.2, 0.0), "start": (14.5, 2.5, 1.5), "stop": (14.5, 20.5, nz - 2.5)},
+    ]
+    return s
+
+
+def _upml_sheet(axis, thick=0):
+    """all components on a sheet (or slab) normal to `axis`, along z over all chunks, UPML cells included"""
+    s = _graded(40, 8)
+    L = s["lines"]
+    lo, hi = [l[3] for l in L], [l[-4] for l in L]
+    lo[axis], hi[axis] = L[axis][17], L[axis][17 + thick]
+    s["excitations"] = [{"type": 0, "val": (1.0, -0.5, 0.25), "start": tuple(lo), "stop": tuple(hi)},
+                        {"type": 2, "val": (0.0, 0.3, 0.1), "start": tuple(lo), "stop": tuple(hi)}]
+    return s
+
+
 CASES = [
     # scene, tile (columns x, y, planes; None: the automatic one), layout, steps
     ("cavity_5x4x3", lambda: _cavity(5, 4, 3), None, "auto", 9),
@@ -54,6 +78,10 @@ CASES = [
     ("upml_40_plain", lambda: _graded(40, 8), "16,12,7", "plain", 61),
     ("upml_45_pml6", lambda: _graded(45, 6), None, "compressed", 60),
     ("upml_40_pml6_one_plane", lambda: _graded(40, 6), "40,9,1", "compressed", 40),
+    ("columns_30x24x22", lambda: _columns(30, 24, 22), "11,9,6", "plain", 31),
+    ("columns_30x24x22_tables", lambda: _columns(30, 24, 22), "11,9,6", "compressed", 30),
+    ("upml_40_x_sheet", lambda: _upml_sheet(0), "16,12,7", "compressed", 41),
+    ("upml_40_y_slab", lambda: _upml_sheet(1, 2), "13,11,9", "plain", 40),
     ("wires_36", lambda: scenes.wire_antenna(36, 100), "11,36,36", "auto", 80),
 ]
 
