@@ -156,9 +156,10 @@ int ems_steady_state(ems_engine* h, double* last_max_diff, unsigned* evaluations
  * faces included; on rows of at least 64 quads it runs in 64 x 4 quad tiles
  * that take neighbour voltages from LDS and adjacent lanes, and runs the
  * pre and post hooks of Mur faces on x = 0 and x = Nx-1 itself.
- * mode: -1 automatic (form 3 on meshes without UPML whose rows hold at
- * least 64 quads, where every active extension has a sweep form and the
- * second field copy fits in device memory; two half steps otherwise),
+ * mode: -1 automatic (pairs of timesteps where ems_get_pair tells; steps
+ * outside pairs in form 3 on meshes without UPML whose rows hold at least 64
+ * quads, where every active extension has a sweep form and the second field
+ * copy fits in device memory; in two half steps otherwise),
  * 0 two half steps, 1 LDS sweep, 2 column sweep, 3 quad column sweep
  * (ems_init then fails with EMS_E_ARG when the engine has no such form). */
 int ems_set_fused(ems_engine* h, int mode);
@@ -179,12 +180,15 @@ int ems_set_quad(ems_engine* h, int mode);
 /* on: 1 when the half steps run quads; zdepth: their z planes per workgroup */
 int ems_get_quad(const ems_engine* h, int* on, unsigned* zdepth);
 
-/* Two timesteps in one launch (k_pair), the automatic step of two-half-step
- * engines whose only extensions are UPML and sources (step form and lane
- * width both automatic, second copies of fields and fluxes fit): wherever no
- * probe or dump samples the state between them; other steps run the two half
- * steps.  Results are bit-identical.  on: 1 when active; tile: columns along
- * x and y and planes of a workgroup; launches: pairs advanced so far. */
+/* Two timesteps in one launch (k_pair), the automatic step of engines whose
+ * only extensions are UPML and sources (step form and lane width both
+ * automatic, second copies of fields and fluxes fit with 1 GiB to spare; with
+ * UPML from a million cells on): wherever no probe or dump samples the state
+ * between them; other steps run singly.  Results are bit-identical.  Device
+ * memory that the engine or its adjoint needs later and that is not free is
+ * taken from the second copies: single steps from then on, as in a batch.
+ * on: 1 when active; tile: columns along x and y and planes of a workgroup;
+ * launches: pairs advanced so far. */
 int ems_get_pair(const ems_engine* h, int* on, unsigned tile[3], unsigned* launches);
 
 /* Active layouts and table sizes (known after ems_init for the UPML part):

@@ -2091,13 +2091,13 @@ __global__ __launch_bounds__(kBlock, 3) void k_step4t(const Step4Args ag, const 
 // in flight.  Hence state n is loaded two planes ahead, and coefficients stay
 // in registers until a column's table entry changes.  With loads one plane
 // ahead 82 us per step at 253 x 209 x 178 and 321 us at 256^3 with UPML; as
-// it is 56 and 220 us, against 171 and 315 us in two half steps (device time
-// per step; 168 and 76 G cells/s, 4.2 and 2.3 TB/s of 50 bytes a cell and 52 a
-// UPML position per launch).  Plain stores: non-temporal ones leave the cache
+// it is 56 and 218 us, against 149 to 174 and 315 us in two half steps (device
+// time per step; 168 and 77 G cells/s, 4.2 and 2.3 TB/s of 50 bytes a cell and
+// 52 a UPML position per launch).  Plain stores: non-temporal ones leave the cache
 // lines shared by neighbouring tiles to be merged in memory (237 us at 256^3).
 // ---------------------------------------------------------------------------
 constexpr unsigned kPairMax = 1024;      // threads of a workgroup (columns of its tile)
-constexpr unsigned kPairMaxPml = 512;    // with UPML, whose fluxes and coefficients take 40 registers more
+constexpr unsigned kPairMaxPml = 512;    // with UPML: 202 to 237 registers, without 124 to 128
 constexpr unsigned kLdsBytes = 160u * 1024u;   // of a CU
 constexpr unsigned kPairLds = 18;        // floats of LDS per column: 3 fields x 3 components x 2 planes
 
@@ -5189,12 +5189,15 @@ static const void* pair_kernel(const ems_engine* h, bool lt)
 // detection have hooks between the half steps), where neither the step form
 // nor the lane width was asked for, 32-bit byte offsets reach every cell and
 // the second copy of fields and fluxes fits with 1 GiB to spare.  With UPML
-// from a million cells on: per step 32.3 -> 24.8 us at 109 x 97 x 131, 60 ->
-// 49 us at 160 x 150 x 140, 315 -> 220 us at 256^3, but 20.9 -> 21.9 us at
-// 90^3 and 10.5 -> 13.4 us at 64^3, where a workgroup sweeps few planes and
-// most of them are graded.  Without UPML at every size: 7.2 -> 5.6 us at
-// 64^3, 34.5 -> 17.3 us at 140^3, 96 -> 57 us at 253 x 209 x 178 (plain
-// accesses; 170 us as it ran).
+// from a million cells on: per step 31.8 -> 24.4 us at 109 x 97 x 131, 63.5 ->
+// 44.5 us at 160 x 150 x 140, 315 -> 218 us at 256^3, but 10.5 -> 12.8 us at
+// 64^3, where a workgroup sweeps few planes and most of them are graded; equal
+// at 80^3 (16.9 us), 20.6 -> 18.7 us at 90^3.  Flat and long meshes above the
+// line: 400 x 400 x 24 78.6 -> 79.5 us, 24 x 400 x 400 93 -> 71, 400 x 24 x 400
+// 75 -> 64, 1000 x 1000 x 20 520 -> 402, 50 x 50 x 500 33.9 -> 24.6, 300 x 60 x
+// 60 25.5 -> 23.6.  Without UPML at every size: 7.1 -> 5.6 us at 64^3, 34.5 ->
+// 14.4 us at 140^3, 103 -> 56 us at 253 x 209 x 178 (plain accesses; 149 to
+// 174 us as it ran), also from 4^3 on and for plates and rods.
 constexpr unsigned long long kPairUpmlCells = 1000000;
 static int build_pair(ems_engine* h)
 {
