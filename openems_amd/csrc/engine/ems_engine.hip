@@ -5198,7 +5198,17 @@ static const void* pair_kernel(const ems_engine* h, bool lt)
 // 60 25.5 -> 23.6.  Without UPML at every size: 7.1 -> 5.6 us at 64^3, 34.5 ->
 // 14.4 us at 140^3, 103 -> 56 us at 253 x 209 x 178 (plain accesses; 149 to
 // 174 us as it ran), also from 4^3 on and for plates and rods.
-constexpr unsigned long long kPairUpmlCells = 1000000;
+// Sources in a volume with UPML below four million cells: a pair's updates take
+// a column's entries of a plane one after another, the current sources of half
+// steps have a launch of their own.  Blocks of 0.3 of the lines along each axis,
+// half steps against pairs: three components 51 : 72 us at 110 x 105 x 100, 109
+// : 128 at 160 x 150 x 140, 825 : 326 at 256^3; one component 36 : 38, 80 : 68,
+// 514 : 244; currents of three components 31 : 67 at 110 x 105 x 100, of one 30
+// : 37, 67 : 70 and 320 : 236.  Sheets hold fewer entries and gain (two
+// components, 109 x 97 x 131: 106 : 43 normal to x, 103 : 46 to y).  So half
+// steps where the voltage entries and twice the current entries exceed a 25th
+// of the cells.
+constexpr unsigned long long kPairUpmlCells = 1000000, kPairVolumeCells = 4000000;
 static int build_pair(ems_engine* h)
 {
     h->pair = false;
@@ -5206,7 +5216,9 @@ static int build_pair(ems_engine* h)
     bool on = (!h->fused || h->fused == 3) && h->fused_req == -1 && h->quad_req == -1 && h->mur.empty() &&
               h->lor.empty() && h->rlc.empty() && !h->has_ss && N[0] < 65535 && N[1] < 65535 && N[2] < 65535 &&
               N[0] >= 4 && N[1] >= 4 && N[2] >= 2 && h->cs < (1ull << 30) && h->pmlV.npos < (1ull << 30);
-    bool big = !h->pmlV.n || (unsigned long long)h->g.plane * N[2] >= kPairUpmlCells;
+    const unsigned long long cells = (unsigned long long)h->g.plane * N[2];
+    const unsigned long long entries = (unsigned long long)h->exc[0].K + 2ull * h->exc[1].K;
+    bool big = !h->pmlV.n || (cells >= kPairUpmlCells && (cells >= kPairVolumeCells || 25ull * entries <= cells));
     for (int c = 0; c < 2; ++c) on = on && h->exc[c].host.size() == h->exc[c].K && h->exc[c].K < kSingle;
     if (const char* e = std::getenv("EMS_PAIR")) big = std::atoi(e) != 0;
     if (!on || !big) return 0;

@@ -158,6 +158,17 @@ def test_pair_policy(gpu, monkeypatch):
         eng = EngineHIP(op, **kw)
         assert eng.pair()[0] == want, (op.N, kw)
         eng.close()
+    # UPML above a million cells: a sheet, a block of voltages, of currents half as many
+    for lo, hi, typ, want in ((50, 50, 0, 1), (34, 69, 0, 0), (38, 65, 0, 1), (38, 65, 2, 0)):
+        s = scenes.upml_bricks(104, 100, nbricks=4, dump=False)
+        x, y, z = s["lines"]
+        a, b = (x[lo], y[34], z[34]), (x[hi], y[69], z[69])
+        s["excitations"] = [{"type": typ, "val": (0.0, 0.0, 1.0), "start": a, "stop": b}]
+        op = Operator(s)
+        entries = len(op.excitation(bool(typ))["dir"]) * (2 if typ else 1)
+        eng = EngineHIP(op)
+        assert eng.pair()[0] == want == (25 * entries <= 104 ** 3), (lo, hi, typ, entries)
+        eng.close()
 
 
 def test_sheet_source_over_many_tiles(gpu, monkeypatch):
