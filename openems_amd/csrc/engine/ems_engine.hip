@@ -6727,6 +6727,7 @@ static int set_field(ems_engine* h, float* d, float* alt, const float* in)
     int rc = upload_nijk(h, d, in);
     if (rc || !alt) return rc;
     // the fused step's second buffer must agree on the cells a step leaves alone
+    // (a pair of timesteps leaves none alone)
     HIPCHK(hipMemcpy(alt, d, 3 * h->cs * sizeof(float), hipMemcpyDeviceToDevice));
     HIPCHK(hipDeviceSynchronize());
     return 0;
@@ -6736,11 +6737,11 @@ int ems_get_volt(ems_engine* h, float* out) { return h ? get_field(h, h->V, out)
 int ems_get_curr(ems_engine* h, float* out) { return h ? get_field(h, h->I, out) : fail(EMS_E_ARG, "null handle"); }
 int ems_set_volt(ems_engine* h, const float* in)
 {
-    return h ? set_field(h, h->V, h->V_alt, in) : fail(EMS_E_ARG, "null handle");
+    return h ? set_field(h, h->V, h->fused ? h->V_alt : nullptr, in) : fail(EMS_E_ARG, "null handle");
 }
 int ems_set_curr(ems_engine* h, const float* in)
 {
-    return h ? set_field(h, h->I, h->I_alt, in) : fail(EMS_E_ARG, "null handle");
+    return h ? set_field(h, h->I, h->fused ? h->I_alt : nullptr, in) : fail(EMS_E_ARG, "null handle");
 }
 
 // one component's box [s, s+n) as x-fastest planes, through pitched copies
@@ -6806,7 +6807,7 @@ int ems_write_field(ems_engine* h, int is_curr, int comp, const unsigned start[3
     std::vector<float> stage(cnt);
     const int c0 = comp < 0 ? 0 : comp, c1 = comp < 0 ? 2 : comp;
     // the fused step's second buffer must agree on the cells a step leaves alone
-    float* bufs[2] = {is_curr ? h->I : h->V, is_curr ? h->I_alt : h->V_alt};
+    float* bufs[2] = {is_curr ? h->I : h->V, !h->fused ? nullptr : is_curr ? h->I_alt : h->V_alt};
     for (int c = c0; c <= c1; ++c) {
         const float* src = in + (size_t)(c - c0) * cnt;
         for (unsigned x = 0; x < n[0]; ++x)

@@ -304,3 +304,29 @@ def test_pairs_beside_quad_sweeps(gpu, monkeypatch, shape, interval, curr, graph
     half = len(out) // 2
     for a, b in zip(out[:half], out[half:]):
         assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
+
+
+def test_setting_a_field_does_not_wait_for_other_engines(gpu, monkeypatch):
+    """Fields of a small engine are set while a large one advances."""
+    monkeypatch.delenv("EMS_PAIR", raising=False)
+    small, large = EngineHIP(Operator(_cavity(20, 18, 16))), EngineHIP(Operator(_cavity(250, 240, 250)))
+    assert small.pair()[0] == 1
+    rng = np.random.default_rng(2)
+    v = rng.standard_normal((3,) + tuple(small.N)).astype(np.float32)
+    large.IterateTS(64)                    # its chunk is captured
+    small.set_volt(v)
+    print("case set a field beside a running engine", flush=True)
+    large.set_async(True)
+    t = time.perf_counter()
+    large.IterateTS(6400)
+    small.set_volt(2 * v)
+    small.write_field(True, (1, 2, 3), (2, 3, 4), v[:, :2, :2, :2])
+    t_set = time.perf_counter() - t
+    large.sync()
+    t_all = time.perf_counter() - t
+    print("set after %.3f s, all done after %.3f s" % (t_set, t_all), flush=True)
+    assert t_set < 0.5 * t_all
+    assert np.array_equal(small.get_volt(), 2 * v)
+    assert np.array_equal(small.read_field(True, (1, 2, 3), (2, 3, 4)), v[:, :2, :2, :2])
+    small.close()
+    large.close()
