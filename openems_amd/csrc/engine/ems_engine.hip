@@ -5333,7 +5333,7 @@ static int build_pair(ems_engine* h)
         if ((rc = h->alloc(&h->flux_alt[side], 3 * np))) return rc;
         HIPCHK(hipMemset(h->flux_alt[side], 0, 3 * np * sizeof(float)));
     }
-    HIPCHK(hipDeviceSynchronize());
+    HIPCHK(hipStreamSynchronize(nullptr));       // the fills; not other engines' streams
     h->numts_alt = h->numts_dev + 2;
     h->V_base = h->V;
     h->pair = true;

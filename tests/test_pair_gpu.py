@@ -330,3 +330,23 @@ def test_setting_a_field_does_not_wait_for_other_engines(gpu, monkeypatch):
     assert np.array_equal(small.read_field(True, (1, 2, 3), (2, 3, 4)), v[:, :2, :2, :2])
     small.close()
     large.close()
+
+
+def test_creating_an_engine_does_not_wait_for_others(gpu, monkeypatch):
+    """An engine with pairs is set up while a large one advances."""
+    monkeypatch.setenv("EMS_PAIR", "1")
+    large, op = EngineHIP(Operator(_cavity(250, 240, 250))), Operator(_graded(40, 8))
+    EngineHIP(op).close()
+    large.IterateTS(64)
+    print("case engine set up beside a running one", flush=True)
+    large.set_async(True)
+    t = time.perf_counter()
+    large.IterateTS(6400)
+    eng = EngineHIP(op)
+    t_made = time.perf_counter() - t
+    large.sync()
+    t_all = time.perf_counter() - t
+    print("made after %.3f s, all done after %.3f s" % (t_made, t_all), flush=True)
+    assert eng.pair()[0] == 1 and t_made < 0.5 * t_all
+    eng.close()
+    large.close()
